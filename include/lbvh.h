@@ -95,10 +95,12 @@ int lbvh_get_div_mode(const lbvh_ctx *ctx);
  * are validated; results do not depend on them. */
 typedef enum {
   LBVH_TUNE_TREE_TILE = 0, /* leaves per block of the fused up pass: 256|512|1024 */
-  LBVH_TUNE_SORT_BITS = 1  /* digit width of the builds' sort: 8 (4 passes
-                              over the 30-bit Morton keys) or 10 (3 passes);
-                              the reference uses 2-bit digits,
-                              radix-sort.js:486 */
+  LBVH_TUNE_SORT_BITS = 1  /* digit width of the builds' radix sort: 8 (4
+                              passes over the 30-bit Morton keys) or 10 (3
+                              passes); the reference uses 2-bit digits,
+                              radix-sort.js:486.  Not fixed, builds and
+                              sorts of at most 2^18 merge sorted tiles
+                              instead of radix passes */
 } lbvh_tunable;
 /* set_tuning fixes a value for every size (value 0: no fixed value, builds
  * use the autotuned table, else the size-based default: tree tile 1024, and
@@ -177,7 +179,8 @@ int lbvh_aabb_morton(lbvh_ctx *ctx, const float *tri, uint32_t n,
  * 10 bits (10, 10, 10, 2) when LBVH_TUNE_SORT_BITS is fixed at 10 (the
  * autotuned table is for the builds' 30-bit keys).  Destructive like the
  * sorted keys replace `keys`; idx_out[j] is the input position of the key
- * now at j. */
+ * now at j.  At most 2^18 keys are sorted by merging sorted tiles unless the
+ * width is fixed; the result is the same. */
 int lbvh_sort(lbvh_ctx *ctx, uint32_t *keys, int32_t *idx_out, uint32_t n);
 
 /* Replaces initRadixTreeKernel(device).execute(sortedKeyBuf, N)

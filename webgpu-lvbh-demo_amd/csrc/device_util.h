@@ -161,6 +161,64 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v,
   return pre + x - v;
 }
 
+// ---- bounds reductions --------------------------------------------------------
+
+// DPP controls of a wave reduction: row shifts right, then the broadcasts of
+// lane 15 and lane 31 into the rows above.  The result is lane 63's.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ float dpp_or(float v, float other) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(
+      __float_as_int(other), __float_as_int(v), kCtrl, kRows, 0xf, false));
+}
+__device__ __forceinline__ float wave_min(float v) {
+  v = fminf(v, dpp_or<0x111, 0xf>(v, INFINITY));
+  v = fminf(v, dpp_or<0x112, 0xf>(v, INFINITY));
+  v = fminf(v, dpp_or<0x114, 0xf>(v, INFINITY));
+  v = fminf(v, dpp_or<0x118, 0xf>(v, INFINITY));
+  v = fminf(v, dpp_or<0x142, 0xa>(v, INFINITY));
+  v = fminf(v, dpp_or<0x143, 0xc>(v, INFINITY));
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+__device__ __forceinline__ float wave_max(float v) { return -wave_min(-v); }
+
+// Block-wide min/max of 6 values (up to 1,024 threads); result valid in
+// thread 0.
+__device__ __forceinline__ void block_minmax(float v[6]) {
+  __shared__ float s[16][6];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    v[c] = wave_min(v[c]);
+    v[3 + c] = wave_max(v[3 + c]);
+  }
+  if (lane == 0)
+    for (int c = 0; c < 6; ++c) s[wave][c] = v[c];
+  __syncthreads();
+  if (wave == 0) {  // lane w takes wave w's values
+    const int w = lane < (int)(blockDim.x >> 6) ? lane : 0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      v[c] = wave_min(s[w][c]);
+      v[3 + c] = wave_max(s[w][3 + c]);
+    }
+  }
+  __syncthreads();
+}
+
+// Folds the bounds partials of `blocks` blocks (min.xyz, max.xyz in w of
+// thread 0).  Every thread of the block must call it.
+__device__ __forceinline__ void fold_partials(
+    const float4 *__restrict__ partials, uint32_t blocks, float w[6]) {
+  w[0] = w[1] = w[2] = INFINITY;
+  w[3] = w[4] = w[5] = -INFINITY;
+  for (uint32_t b = threadIdx.x; b < blocks; b += blockDim.x) {
+    const float4 lo = partials[2 * b], hi = partials[2 * b + 1];
+    w[0] = fminf(w[0], lo.x); w[1] = fminf(w[1], lo.y); w[2] = fminf(w[2], lo.z);
+    w[3] = fmaxf(w[3], hi.x); w[4] = fmaxf(w[4], hi.y); w[5] = fmaxf(w[5], hi.z);
+  }
+  block_minmax(w);
+}
+
 // ---- Morton keys (aabb-z-idx.js:192-208) ------------------------------------
 //
 // Shared by the single-mesh and the batched kernels so that both produce the

@@ -11,40 +11,6 @@
 
 namespace lbvh {
 
-__device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
-  return v;
-}
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
-}
-
-// Block-wide min/max of 6 values (up to 1,024 threads); result valid in
-// thread 0.
-__device__ void block_minmax(float v[6]) {
-  __shared__ float s[16][6];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    v[c] = wave_min(v[c]);
-    v[3 + c] = wave_max(v[3 + c]);
-  }
-  if (lane == 0)
-    for (int c = 0; c < 6; ++c) s[wave][c] = v[c];
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < (int)(blockDim.x >> 6); ++w)
-      for (int c = 0; c < 3; ++c) {
-        v[c] = fminf(v[c], s[w][c]);
-        v[3 + c] = fmaxf(v[3 + c], s[w][3 + c]);
-      }
-  }
-  __syncthreads();
-}
-
 // Scene bounds: fp32 min/max over all vertex coordinates.  Each block
 // reduces a share of the triangles into partials[2*b, 2*b+1]; k_bounds_final
 // (one block, launched next) folds the partials into ctl->bounds.  No atomics
@@ -103,20 +69,6 @@ __global__ __launch_bounds__(kMapThreads) void k_bounds(
     partials[2 * blockIdx.x] = make_float4(v[0], v[1], v[2], 0.0f);
     partials[2 * blockIdx.x + 1] = make_float4(v[3], v[4], v[5], 0.0f);
   }
-}
-
-// Folds the bounds partials of `blocks` blocks (min.xyz, max.xyz in w of
-// thread 0).  Every thread of the block must call it.
-__device__ void fold_partials(const float4 *__restrict__ partials,
-                              uint32_t blocks, float w[6]) {
-  w[0] = w[1] = w[2] = INFINITY;
-  w[3] = w[4] = w[5] = -INFINITY;
-  for (uint32_t b = threadIdx.x; b < blocks; b += blockDim.x) {
-    const float4 lo = partials[2 * b], hi = partials[2 * b + 1];
-    w[0] = fminf(w[0], lo.x); w[1] = fminf(w[1], lo.y); w[2] = fminf(w[2], lo.z);
-    w[3] = fmaxf(w[3], hi.x); w[4] = fmaxf(w[4], hi.y); w[5] = fmaxf(w[5], hi.z);
-  }
-  block_minmax(w);
 }
 
 // One block of kFoldThreads: two partials per thread at the largest grid,

@@ -47,6 +47,7 @@ struct lbvh_ctx {
   int tune_tile[33] = {0};       // autotuned tree tile per log2 size bucket
   int sort_bits = kRadixBits;    // sort digit width (8 or 10)
   bool sort_bits_fixed = false;
+  bool tuning = false;           // lbvh_autotune is timing its variants
   int tune_bits[33] = {0};       // autotuned digit width per size bucket
   std::string last_error;
   AllocTable user_allocs;  // buffers handed out by lbvh_alloc
@@ -462,6 +463,12 @@ int bits_for(const lbvh_ctx *ctx, uint32_t n) {
                    untuned_bits(n));
 }
 
+// Whether a single-mesh sort of n keys merges sorted tiles; a fixed digit
+// width asks for the radix passes.
+bool merge_sorted(const lbvh_ctx *ctx, uint32_t n) {
+  return n <= kMergeSortMax && !(ctx->sort_bits_fixed && !ctx->tuning);
+}
+
 // The key buffers of each pass of a sort from `in` to `out`: each pass reads
 // one buffer and writes another.  An even number of passes runs
 // in -> tmp -> out -> tmp -> out (`in` may equal `out`); an odd one runs
@@ -609,6 +616,31 @@ int check_build_args(lbvh_ctx *ctx, const float *tri, uint32_t n,
                            {perm_out, 4ull * n, "permutation output"}});
 }
 
+// Morton keys and their radix passes: n triangles' keys sorted into skeys and
+// perm.  from_ctl: GPU bounds (the centres in S.cen when n > 1, `parts`
+// partials still to fold), else those in p.
+void build_radix(lbvh_ctx *ctx, const BuildScratch &S, const float4 *t4,
+                 uint32_t n, const MortonParams &p, bool from_ctl,
+                 uint32_t parts, uint32_t *tmp, uint32_t *skeys,
+                 int32_t *perm, int bits) {
+  uint32_t *keys = S.keys_a;
+  {
+    StageScope sc(ctx, LBVH_STAGE_MORTON);
+    uint32_t *cnt = n > 1 ? S.digits : nullptr;
+    if (S.cen)
+      launch_morton_cen(S.cen, n, p.div_mode, keys, ctx->ctl, cnt, bits,
+                        ctx->stream, S.partials, parts);
+    else
+      launch_aabb_morton(t4, n, p, from_ctl, nullptr, keys, ctx->ctl,
+                         ctx->stream, cnt, bits);
+  }
+  if (n > 1)
+    run_sort(ctx, S.digits, keys, tmp, skeys, nullptr, S.idx_b, perm, n, true,
+             bits);
+  else
+    launch_single_key(keys, skeys, perm, ctx->stream);
+}
+
 // Enqueues the whole build of n >= 1 triangles: bounds (unless given),
 // Morton keys with the first pass's digit counts, the sort, the
 // agglomeration levels.  Enqueues kernels only: no allocation, copy or
@@ -617,42 +649,45 @@ void build_pipeline(lbvh_ctx *ctx, const BuildScratch &S, const float *tri,
                     uint32_t n, const float *bounds_host, void *bvh_out,
                     float *tri_out, uint32_t *sorted_keys_out,
                     int32_t *perm_out, int bits, int tile) {
-  const bool sort = n > 1;
   // GPU bounds: the bounds pass also writes the box centres, and the Morton
   // pass reads those (12 bytes per triangle) instead of the triangles
   const bool use_cen = S.cen != nullptr;
   const float4 *t4 = reinterpret_cast<const float4 *>(tri);
-  uint32_t *keys = S.keys_a;
-  uint32_t *tmp = S.keys_b;
-  uint32_t *skeys = sorted_keys_out ? sorted_keys_out : keys;
-  // an odd number of passes ends in the other buffer: sort into keys_b
-  if (sort && sort_passes(bits) % 2 && skeys == keys) std::swap(skeys, tmp);
+  uint32_t *skeys = sorted_keys_out ? sorted_keys_out : S.keys_a;
   int32_t *perm = perm_out ? perm_out : S.idx_a;
+  const bool merge = merge_sorted(ctx, n);
+  // a mesh of one sort tile: the tile sort takes its bounds too
+  const bool whole = merge && !bounds_host && n <= (uint32_t)kMsTile;
   MortonParams p{};
   uint32_t parts = 0;  // bounds partials the Morton pass folds itself
   if (bounds_host) {
     p = morton_params(ctx, bounds_host);
   } else {
     p.div_mode = ctx->div_mode;
+  }
+  if (!bounds_host && !whole) {
     StageScope sc(ctx, LBVH_STAGE_BOUNDS);
     parts = launch_bounds(t4, n, S.partials, ctx->ctl, ctx->stream, S.cen,
                           use_cen ? kFoldPartialsMax : 0);
   }
-  {
-    StageScope sc(ctx, LBVH_STAGE_MORTON);
-    uint32_t *cnt = sort ? S.digits : nullptr;
-    if (use_cen)
-      launch_morton_cen(S.cen, n, ctx->div_mode, keys, ctx->ctl, cnt, bits,
-                        ctx->stream, S.partials, parts);
-    else
-      launch_aabb_morton(t4, n, p, bounds_host == nullptr, nullptr, keys,
-                         ctx->ctl, ctx->stream, cnt, bits);
+  if (merge) {
+    const MergeKeys src{nullptr, whole ? nullptr : S.cen, t4, S.partials,
+                        parts,   whole,                   ctx->ctl, p};
+    {
+      StageScope sc(ctx, LBVH_STAGE_MORTON);
+      launch_tile_sort(src, n, S.keys_b, S.idx_b, skeys, perm, S.digits,
+                       ctx->stream);
+    }
+    StageScope sc(ctx, LBVH_STAGE_SORT0);
+    launch_merge_rounds(src, n, S.keys_b, S.idx_b, skeys, perm, S.digits,
+                        ctx->stream);
+  } else {
+    uint32_t *tmp = S.keys_b;
+    // an odd number of passes ends in the other buffer: sort into keys_b
+    if (n > 1 && sort_passes(bits) % 2 && skeys == S.keys_a) std::swap(skeys, tmp);
+    build_radix(ctx, S, t4, n, p, bounds_host == nullptr, parts, tmp, skeys,
+                perm, bits);
   }
-  if (sort)
-    run_sort(ctx, S.digits, keys, tmp, skeys, nullptr, S.idx_b, perm, n, true,
-             bits);
-  else
-    launch_single_key(keys, skeys, perm, ctx->stream);
   run_tree(ctx, S.tree_items, S.tree_counts, tri, skeys, perm, n, tri_out,
            bvh_out, tile);
 }
@@ -986,6 +1021,7 @@ int lbvh_autotune(lbvh_ctx *ctx, uint32_t n_min, uint32_t n_max, int reps,
   const bool bits_were_fixed = ctx->sort_bits_fixed;
   ctx->tree_tile_fixed = true;  // force each variant while timing
   ctx->sort_bits_fixed = true;
+  ctx->tuning = true;
   const int saved_tile = ctx->tree_tile, saved_bits = ctx->sort_bits;
   int out_i = 0;
   st = LBVH_OK;
@@ -1033,6 +1069,7 @@ int lbvh_autotune(lbvh_ctx *ctx, uint32_t n_min, uint32_t n_max, int reps,
       ctx->tune_bits[k] = widths[pick % 2];
     }
   }
+  ctx->tuning = false;
   ctx->tree_tile = saved_tile;
   ctx->sort_bits = saved_bits;
   ctx->tree_tile_fixed = (st == LBVH_OK) ? false : tile_was_fixed;
@@ -1223,6 +1260,16 @@ int lbvh_sort(lbvh_ctx *ctx, uint32_t *keys, int32_t *idx_out, uint32_t n) {
   // 10-bit digits take 4 passes here too, so they run only when fixed.
   const int bits = ctx->sort_bits_fixed ? ctx->sort_bits : kRadixBits;
   if ((st = ensure_sort_scratch(ctx, n, bits))) return st;
+  if (merge_sorted(ctx, n)) {
+    MergeKeys src{};
+    src.keys = keys;
+    uint32_t *kt = static_cast<uint32_t *>(ctx->keys_b.ptr);
+    int32_t *vt = static_cast<int32_t *>(ctx->idx_a.ptr);
+    uint32_t *smp = static_cast<uint32_t *>(ctx->digits.ptr);
+    launch_tile_sort(src, n, kt, vt, keys, idx_out, smp, ctx->stream);
+    launch_merge_rounds(src, n, kt, vt, keys, idx_out, smp, ctx->stream);
+    return check_launch(ctx, "lbvh_sort");
+  }
   run_sort(ctx, static_cast<uint32_t *>(ctx->digits.ptr), keys,
            static_cast<uint32_t *>(ctx->keys_b.ptr), keys,
            static_cast<uint32_t *>(ctx->keys_a.ptr),

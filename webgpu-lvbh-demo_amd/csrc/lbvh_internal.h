@@ -159,6 +159,41 @@ inline uint32_t batch_sort_tiles(uint32_t n) {
 void launch_single_key(const uint32_t *keys, uint32_t *sorted, int32_t *perm,
                        hipStream_t s);
 
+// k_merge_sort.hip
+// A single mesh of at most kMergeSortMax keys is sorted by tiles of kMsTile
+// keys in LDS and rank merges of the tiles, not by radix passes: one merge
+// round up to 32 tiles, two up to 128.  Builds of uniform meshes, merged
+// against the better digit width: 2^12 36 / 54 us, 2^16 47 / 67, 2^17 65 / 81,
+// 2^18 81 / 93 (heightfields: 38 / 56, 52 / 68, 71 / 79, 84 / 90); a third
+// round loses to the radix passes (300,000: 111 / 105).
+constexpr int kMsTileLog = 11;
+constexpr int kMsTile = 1 << kMsTileLog;
+constexpr uint32_t kMergeSortMax = 128u << kMsTileLog;
+// The keys of a merge sort: given (any u32; `keys` may be the output), or
+// Morton keys made by the tile sort -- from the centres launch_bounds wrote
+// with the bounds folded from `parts` partials (0: those in ctl), from the
+// triangles with the bounds in p, or (whole: n <= kMsTile) from the triangles
+// with the bounds of the one tile.
+struct MergeKeys {
+  const uint32_t *keys;
+  const float *cen;
+  const float4 *tri;
+  const float4 *partials;
+  uint32_t parts;
+  int whole;
+  const Ctl *ctl;
+  MortonParams p;
+};
+// The tile sort, then the merge rounds, both given the same buffers: the
+// sorted keys and their input positions end in keys_out and idx_out.
+// samples: n / 16 + 2 words (a sort's digit counts and offsets are more).
+void launch_tile_sort(const MergeKeys &src, uint32_t n, uint32_t *keys_tmp,
+                      int32_t *idx_tmp, uint32_t *keys_out, int32_t *idx_out,
+                      uint32_t *samples, hipStream_t s);
+void launch_merge_rounds(const MergeKeys &src, uint32_t n, uint32_t *keys_tmp,
+                         int32_t *idx_tmp, uint32_t *keys_out,
+                         int32_t *idx_out, uint32_t *samples, hipStream_t s);
+
 // k_tree.hip
 // The per-stage radix tree (parents array) in three launches over 4,096-gap
 // tiles; scratch of radix_tree_scratch_bytes(n) (spine records, per-tile
