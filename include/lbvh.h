@@ -94,7 +94,10 @@ int lbvh_get_div_mode(const lbvh_ctx *ctx);
  * digit sizes are constants, e.g. WG_SIZE = 64 at aabb-z-idx.js:4).  Values
  * are validated; results do not depend on them. */
 typedef enum {
-  LBVH_TUNE_TREE_TILE = 0, /* leaves per block of the fused up pass: 256|512|1024 */
+  LBVH_TUNE_TREE_TILE = 0, /* leaves per block of the fused up pass:
+                              256|512|1024.  Not fixed, builds and refits of
+                              at most 2^21 triangles take tiles of their own
+                              (256 leaves, no climb) */
   LBVH_TUNE_SORT_BITS = 1  /* digit width of the builds' radix sort: 8 (4
                               passes over the 30-bit Morton keys) or 10 (3
                               passes); the reference uses 2-bit digits,

@@ -181,6 +181,18 @@ __device__ __forceinline__ float wave_min(float v) {
 }
 __device__ __forceinline__ float wave_max(float v) { return -wave_min(-v); }
 
+// Inclusive prefix sum over the wave's lanes.
+__device__ __forceinline__ uint32_t wave_scan_add(uint32_t x) {
+  int v = (int)x;
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+  return (uint32_t)v;
+}
+
 // Block-wide min/max of 6 values (up to 1,024 threads); result valid in
 // thread 0.
 __device__ __forceinline__ void block_minmax(float v[6]) {

@@ -458,6 +458,17 @@ int untuned_bits(uint32_t n) {
   return wide ? kWideBits : kRadixBits;
 }
 
+// The tree levels of an n-triangle mesh: leaf tile, and whether they are
+// k_forest.hip's (small meshes, unless the tile is fixed).
+struct TreePlan {
+  int tile;
+  bool forest;
+};
+TreePlan tree_plan(const lbvh_ctx *ctx, uint32_t n) {
+  if (n <= kForestMax && !ctx->tree_tile_fixed) return {kForestTile, true};
+  return {tile_for(ctx, n), false};
+}
+
 int bits_for(const lbvh_ctx *ctx, uint32_t n) {
   return tuned_for(ctx->sort_bits, ctx->sort_bits_fixed, ctx->tune_bits, n,
                    untuned_bits(n));
@@ -549,18 +560,26 @@ void run_sort(lbvh_ctx *ctx, uint32_t *digits, const uint32_t *in,
 // then the item levels above them, each level its own profiling stage.
 void run_tree(lbvh_ctx *ctx, int4 *items, uint32_t *counts, const float *tri,
               const uint32_t *skeys, const int32_t *perm, uint32_t n,
-              float *tri_out, void *bvh_out, int tile) {
+              float *tri_out, void *bvh_out, const TreePlan &plan) {
   uint32_t grid[kMaxTreeLevels];
-  const int levels = tree_levels(n, tile, grid);
+  const int levels = tree_levels(n, plan.tile, grid);
+  const float4 *t4 = reinterpret_cast<const float4 *>(tri);
+  float4 *o4 = reinterpret_cast<float4 *>(tri_out);
+  float4 *nodes = static_cast<float4 *>(bvh_out);
   uint64_t base = 0, prev = 0;
   for (int L = 0; L < levels; ++L) {
     StageScope sc(ctx, L ? LBVH_STAGE_TREE_TOP : LBVH_STAGE_TREE);
-    launch_tree_level(L, tile, grid[L], reinterpret_cast<const float4 *>(tri),
-                      skeys, perm, n, reinterpret_cast<float4 *>(tri_out),
-                      items + kItemInt4 * kTreeFrontier * prev, counts + prev,
-                      L ? grid[L - 1] : 0u, items + kItemInt4 * kTreeFrontier * base,
-                      counts + base, static_cast<float4 *>(bvh_out), ctx->ctl,
-                      TreeSegs{}, ctx->stream);
+    const int4 *items_in = items + kItemInt4 * kTreeFrontier * prev;
+    int4 *items_out = items + kItemInt4 * kTreeFrontier * base;
+    const uint32_t below = L ? grid[L - 1] : 0u;
+    if (plan.forest)
+      launch_forest_level(L, grid[L], t4, skeys, perm, n, o4, items_in,
+                          counts + prev, below, items_out, counts + base,
+                          nodes, ctx->ctl, ctx->stream);
+    else
+      launch_tree_level(L, plan.tile, grid[L], t4, skeys, perm, n, o4, items_in,
+                        counts + prev, below, items_out, counts + base, nodes,
+                        ctx->ctl, TreeSegs{}, ctx->stream);
     prev = base;
     base += grid[L];
   }
@@ -648,7 +667,7 @@ void build_radix(lbvh_ctx *ctx, const BuildScratch &S, const float4 *t4,
 void build_pipeline(lbvh_ctx *ctx, const BuildScratch &S, const float *tri,
                     uint32_t n, const float *bounds_host, void *bvh_out,
                     float *tri_out, uint32_t *sorted_keys_out,
-                    int32_t *perm_out, int bits, int tile) {
+                    int32_t *perm_out, int bits, const TreePlan &plan) {
   // GPU bounds: the bounds pass also writes the box centres, and the Morton
   // pass reads those (12 bytes per triangle) instead of the triangles
   const bool use_cen = S.cen != nullptr;
@@ -689,7 +708,7 @@ void build_pipeline(lbvh_ctx *ctx, const BuildScratch &S, const float *tri,
                 perm, bits);
   }
   run_tree(ctx, S.tree_items, S.tree_counts, tri, skeys, perm, n, tri_out,
-           bvh_out, tile);
+           bvh_out, plan);
 }
 
 // Lays out one build's scratch from `base` (null: sizes only); returns the
@@ -1346,10 +1365,10 @@ int lbvh_build(lbvh_ctx *ctx, const float *tri, uint32_t n,
     return st;
   if ((st = check_bounds(ctx, bounds_host, 1))) return st;
   const int bits = bits_for(ctx, n);
-  const int tile = tile_for(ctx, n);
+  const TreePlan plan = tree_plan(ctx, n);
   const bool use_cen = !bounds_host && n > 1;
   if ((st = ensure_sort_scratch(ctx, n, bits))) return st;
-  if ((st = ensure_tree_scratch(ctx, n, tile))) return st;
+  if ((st = ensure_tree_scratch(ctx, n, plan.tile))) return st;
   if (!bounds_host && (st = ensure_partials(ctx))) return st;
   if (use_cen && (st = ensure(ctx, ctx->cen, 12ull * cen_stride(n), false)))
     return st;
@@ -1364,7 +1383,7 @@ int lbvh_build(lbvh_ctx *ctx, const float *tri, uint32_t n,
   S.partials = static_cast<float4 *>(ctx->partials.ptr);
   S.cen = use_cen ? static_cast<float *>(ctx->cen.ptr) : nullptr;
   build_pipeline(ctx, S, tri, n, bounds_host, bvh_out, tri_out,
-                 sorted_keys_out, perm_out, bits, tile);
+                 sorted_keys_out, perm_out, bits, plan);
   return check_launch(ctx, "lbvh_build");
 }
 
@@ -1386,10 +1405,10 @@ int lbvh_build_static(lbvh_ctx *ctx, const float *tri, uint32_t n,
     return fail(ctx, LBVH_ERR_DEVICE,
                 "the static scratch has no address on this device");
   const int bits = bits_for(ctx, n);
-  const int tile = tile_for(ctx, n);
+  const TreePlan plan = tree_plan(ctx, n);
   BuildScratch S;
   const uint64_t need =
-      layout_build_scratch(n, bits, tile, !bounds_host && n > 1,
+      layout_build_scratch(n, bits, plan.tile, !bounds_host && n > 1,
                            static_cast<char *>(ctx->static_scratch), &S);
   if (need > kStaticScratchBytes)
     return fail(ctx, LBVH_ERR_INVALID_ARGUMENT,
@@ -1400,7 +1419,7 @@ int lbvh_build_static(lbvh_ctx *ctx, const float *tri, uint32_t n,
   const bool prof = ctx->prof;
   ctx->prof = false;
   build_pipeline(ctx, S, tri, n, bounds_host, bvh_out, tri_out,
-                 sorted_keys_out, perm_out, bits, tile);
+                 sorted_keys_out, perm_out, bits, plan);
   ctx->prof = prof;
   return check_launch(ctx, "lbvh_build_static");
 }
@@ -1420,11 +1439,11 @@ int lbvh_refit(lbvh_ctx *ctx, const float *tri, uint32_t n,
                               {bvh_out, 64ull * n, "BVH output"},
                               {tri_out, 48ull * n, "triangle output"}})))
     return st;
-  const int tile = tile_for(ctx, n);
-  if ((st = ensure_tree_scratch(ctx, n, tile))) return st;
+  const TreePlan plan = tree_plan(ctx, n);
+  if ((st = ensure_tree_scratch(ctx, n, plan.tile))) return st;
   run_tree(ctx, static_cast<int4 *>(ctx->tree_items.ptr),
            static_cast<uint32_t *>(ctx->tree_counts.ptr), tri, sorted_keys,
-           perm, n, tri_out, bvh_out, tile);
+           perm, n, tri_out, bvh_out, plan);
   return check_launch(ctx, "lbvh_refit");
 }
 
