@@ -32,26 +32,29 @@ __device__ __forceinline__ V3 v3(int4 v) {
   return {__int_as_float(v.x), __int_as_float(v.y), __int_as_float(v.z)};
 }
 
-// tri_intersect (pathtracer.js:587-619): (normal, t) or t = -1.
-__device__ __forceinline__ float4 tri_intersect(V3 o, V3 d, V3 v0, V3 v1,
-                                                V3 v2) {
+// The distance of tri_intersect (pathtracer.js:587-619), -1 for a miss.
+__device__ __forceinline__ float tri_distance(V3 o, V3 d, V3 v0, V3 v1, V3 v2) {
   const V3 e1 = sub(v1, v0), e2 = sub(v2, v0);
   const V3 pvec = cross(d, e2);
   const float det = dot(e1, pvec);
-  if (fabsf(det) < 1e-10f) return make_float4(-1.f, -1.f, -1.f, -1.f);
+  if (fabsf(det) < 1e-10f) return -1.f;
   const float idet = __fdiv_rn(1.0f, det);
   const V3 tvec = sub(o, v0);
   const float u = __fmul_rn(dot(tvec, pvec), idet);
-  if (u < 0.f || u > 1.f) return make_float4(-1.f, -1.f, -1.f, -1.f);
+  if (u < 0.f || u > 1.f) return -1.f;
   const V3 qvec = cross(tvec, e1);
   const float v = __fmul_rn(dot(d, qvec), idet);
-  if (v < 0.f || __fadd_rn(u, v) > 1.f) return make_float4(-1.f, -1.f, -1.f, -1.f);
-  const V3 nrm = cross(e1, e2);
+  if (v < 0.f || __fadd_rn(u, v) > 1.f) return -1.f;
+  return __fmul_rn(dot(e2, qvec), idet);
+}
+
+// Its normal, taken once per ray for the closest hit.
+__device__ __forceinline__ V3 tri_normal(V3 v0, V3 v1, V3 v2) {
+  const V3 nrm = cross(sub(v1, v0), sub(v2, v0));
   // __builtin_sqrtf is correctly rounded (the default fp32 mode); HIP's
   // __fsqrt_rn maps to the hardware approximation, which is not.
   const float len = __builtin_sqrtf(dot(nrm, nrm));
-  return make_float4(__fdiv_rn(nrm.x, len), __fdiv_rn(nrm.y, len),
-                     __fdiv_rn(nrm.z, len), __fmul_rn(dot(e2, qvec), idet));
+  return {__fdiv_rn(nrm.x, len), __fdiv_rn(nrm.y, len), __fdiv_rn(nrm.z, len)};
 }
 
 // aabb_intersect (pathtracer.js:621-628): entry distance or -1e30.
@@ -68,12 +71,41 @@ __device__ __forceinline__ float aabb_intersect(V3 lo, V3 hi, V3 o, V3 inv) {
 }
 
 constexpr int kRayStack = 64;  // the path tracer's is 32 (pathtracer.js:493)
+constexpr int kRayLds = 24;    // entries of it in LDS; deeper ones are rare
+constexpr int kRayThreads = 64;
+constexpr uint32_t kRayChunk = 64;  // consecutive blocks on one XCD
 
-__global__ __launch_bounds__(kMapThreads) void k_raycast(
+// A step fetches one node or triangle and waits for it, and a frame lasts as
+// long as its longest waves (those that cross dense clusters), so what counts
+// is the latency of a step:
+//   * one fetch for either kind: lanes at a node and lanes at a triangle wait
+//     together, not one after the other;
+//   * the stack's first kRayLds entries are in LDS (an array indexed per lane
+//     is in scratch memory; 24 words per lane leave the CU its 24 waves), in
+//     blocks of one wave, so a finished wave's share is free at once;
+//   * the normal, a square root and three divisions, is taken once at the
+//     end, of the closest hit;
+//   * kRayChunk blocks (4,096 rays) in a row run on one XCD, whose L2 then
+//     holds the nodes they share (1M rays of a frame over 1M triangles 398 ->
+//     317 us).
+// Together 245 -> 181 us for a 512 x 512 frame over 100,000 clustered
+// triangles, 1,000 -> 740 us for 1M scattered rays over 1M.  Dropping popped
+// nodes beyond the closest hit lost (the stack entries double), and so did
+// descending to a leaf per lane before any test, and touching both children
+// ahead.
+__global__ __launch_bounds__(kRayThreads) void k_raycast(
     const int4 *__restrict__ nodes, const int4 *__restrict__ tri, uint32_t n,
     const float4 *__restrict__ rays, uint32_t count, float4 *__restrict__ hits,
     uint32_t max_steps) {
-  const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
+  __shared__ int s_stack[kRayLds][kRayThreads];
+  int deep[kRayStack - kRayLds];
+  const uint32_t tid = threadIdx.x;
+  // chunks of kRayChunk blocks go to the XCDs in turn; the rest as they come
+  constexpr uint32_t kTurn = kXcds * kRayChunk;
+  uint32_t blk = blockIdx.x;
+  if (blk < gridDim.x / kTurn * kTurn)
+    blk = blk / kTurn * kTurn + blk % kXcds * kRayChunk + blk / kXcds % kRayChunk;
+  const uint32_t q = blk * kRayThreads + tid;
   if (q >= count) return;
   const float4 ro = rays[2 * (size_t)q], rd = rays[2 * (size_t)q + 1];
   const V3 o = {ro.x, ro.y, ro.z};
@@ -85,49 +117,51 @@ __global__ __launch_bounds__(kMapThreads) void k_raycast(
   const V3 inv = {__fdiv_rn(1.0f, d.x), __fdiv_rn(1.0f, d.y),
                   __fdiv_rn(1.0f, d.z)};
   float dist = 1e30f;
-  V3 nrm = {0.f, 0.f, 0.f};
-  int stack[kRayStack];
-  int sp = 0;
+  uint32_t hit = 0;  // the closest hit's triangle (dist < 1e30)
+  int sp = 0;        // entries on the stack; -1: the traversal is over
   int node = 0;
   for (uint32_t step = 0; sp >= 0 && step < max_steps; ++step) {
-    if (node < 0) {
-      const uint32_t t = (uint32_t)(-(node + 1));
-      if (t < n) {
-        const float4 h = tri_intersect(o, d, v3(tri[3 * (size_t)t]),
-                                       v3(tri[3 * (size_t)t + 1]),
-                                       v3(tri[3 * (size_t)t + 2]));
-        if (h.w > 0.f && h.w < dist) {
-          nrm = {h.x, h.y, h.z};
-          dist = fminf(h.w, dist);
-        }
+    const bool leaf = node < 0;
+    const uint32_t id = leaf ? (uint32_t)(-(node + 1)) : (uint32_t)node;
+    if (!leaf && id >= n) break;
+    const int4 *at = leaf ? tri + 3 * (size_t)(id < n ? id : 0u)
+                          : nodes + 4 * (size_t)id;
+    const int4 a = at[0], b = at[1], c = at[2], e = at[leaf ? 2 : 3];
+    bool next;  // the next node comes off the stack
+    if (leaf) {
+      const float h = tri_distance(o, d, v3(a), v3(b), v3(c));
+      if (id < n && h > 0.f && h < dist) {
+        dist = h;
+        hit = id;
       }
-      sp -= 1;
-      node = sp >= 0 ? stack[sp] : 0;
+      next = true;
     } else {
-      if ((uint32_t)node >= n) break;
-      const int4 *nd = nodes + 4 * (size_t)node;
-      const int4 a = nd[0], b = nd[1], c = nd[2], e = nd[3];
       const float ld = aabb_intersect(v3(a), v3(b), o, inv);
       const float rdist = aabb_intersect(v3(c), v3(e), o, inv);
       const bool lv = ld != -1e30f && ld < dist;
       const bool rv = rdist != -1e30f && rdist < dist;
+      const bool left = lv && (!rv || ld < rdist);  // the nearer child first
       if (lv && rv) {
-        const int near = ld < rdist ? a.w : c.w;
-        const int far = ld < rdist ? c.w : a.w;
-        if (sp < kRayStack) stack[sp] = far;
+        const int far = left ? c.w : a.w;
+        if (sp < kRayLds) s_stack[sp][tid] = far;
+        else if (sp < kRayStack) deep[sp - kRayLds] = far;
         sp = sp + 1 < kRayStack ? sp + 1 : kRayStack;
-        node = near;
-      } else if (lv) {
-        node = a.w;
-      } else if (rv) {
-        node = c.w;
-      } else {
-        sp -= 1;
-        node = sp >= 0 ? stack[sp] : 0;
       }
+      node = left ? a.w : c.w;
+      next = !lv && !rv;
+    }
+    if (next) {
+      sp -= 1;
+      if (sp >= 0)
+        node = sp < kRayLds ? s_stack[sp][tid] : deep[sp - kRayLds];
     }
   }
   // RayHit: normal facing the ray, dist -1 for a miss (pathtracer.js:572-583)
+  V3 nrm = {0.f, 0.f, 0.f};
+  if (dist < 1e30f) {
+    const int4 *v = tri + 3 * (size_t)hit;
+    nrm = tri_normal(v3(v[0]), v3(v[1]), v3(v[2]));
+  }
   const float s = dot(d, {-nrm.x, -nrm.y, -nrm.z}) > 0.f ? 1.f : -1.f;
   hits[q] = make_float4(s * nrm.x, s * nrm.y, s * nrm.z,
                         dist == 1e30f ? -1.f : dist);
@@ -136,9 +170,9 @@ __global__ __launch_bounds__(kMapThreads) void k_raycast(
 void launch_raycast(const void *nodes, const float *tri, uint32_t n,
                     const float *rays, uint32_t count, float *hits,
                     hipStream_t s) {
-  const uint32_t blocks = (count + kMapThreads - 1) / kMapThreads;
+  const uint32_t blocks = (count + kRayThreads - 1) / kRayThreads;
   const uint64_t cap = 4ull * n + 256;
-  hipLaunchKernelGGL(k_raycast, dim3(blocks ? blocks : 1), dim3(kMapThreads),
+  hipLaunchKernelGGL(k_raycast, dim3(blocks ? blocks : 1), dim3(kRayThreads),
                      0, s, static_cast<const int4 *>(nodes),
                      reinterpret_cast<const int4 *>(tri), n,
                      reinterpret_cast<const float4 *>(rays), count,
