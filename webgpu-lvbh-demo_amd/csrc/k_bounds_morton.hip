@@ -12,8 +12,9 @@
 namespace lbvh {
 
 // Scene bounds: fp32 min/max over all vertex coordinates.  Each block
-// reduces a share of the triangles into partials[2*b, 2*b+1]; k_bounds_final
-// (one block, launched next) folds the partials into ctl->bounds.  No atomics
+// reduces a share of the triangles into partials[2*b, 2*b+1], folded by every
+// block of the kernel that makes the keys, or (without centres) into
+// ctl->bounds by k_bounds_final.  No atomics
 // and no fences: a last-block-finishes counter costs one same-address
 // device-scope atomic (with a cache writeback for its release) per block,
 // which on MI355X serialises across the XCDs.
@@ -71,10 +72,8 @@ __global__ __launch_bounds__(kMapThreads) void k_bounds(
   }
 }
 
-// One block of kFoldThreads: two partials per thread at the largest grid,
-// so the fold waits on one round of loads.
-constexpr int kFoldThreads = 1024;
-__global__ __launch_bounds__(kFoldThreads) void k_bounds_final(
+// One block, a partial per thread.
+__global__ __launch_bounds__(kBoundsBlocks) void k_bounds_final(
     const float4 *__restrict__ partials, uint32_t blocks, Ctl *ctl) {
   float w[6];
   fold_partials(partials, blocks, w);
@@ -184,27 +183,24 @@ __global__ __launch_bounds__(kMapThreads) void k_aabb_morton(
 // compute_aabb_z_idx from the box centres k_bounds wrote (aabb-z-idx.js
 // :192-195 onward; the centre of :191 is already rounded the same way), plus
 // the first sort pass's per-tile digit counts.  One block per sort tile of
-// kTileKeys keys, as k_aabb_morton with cnt.  Bounds from ctl, or (parts != 0) folded by every
-// block from the bounds partials as k_bounds_final folds them, which saves
-// small builds that launch.
+// kTileKeys keys, as k_aabb_morton with cnt; every block folds the bounds
+// partials.
 template <int kBits, int kTileKeys>
 __global__ __launch_bounds__(kMapThreads) void k_morton_cen(
     const float *__restrict__ cen, uint32_t n, int div_mode,
-    uint32_t *__restrict__ keys, const Ctl *ctl, uint32_t *__restrict__ cnt,
+    uint32_t *__restrict__ keys, uint32_t *__restrict__ cnt,
     const float4 *__restrict__ partials, uint32_t parts) {
   constexpr int kR = 1 << kBits;
   __shared__ uint32_t s_hist[kR];
   __shared__ float s_b[8];
   for (int d = threadIdx.x; d < kR; d += kMapThreads) s_hist[d] = 0u;
-  if (parts) {
+  {
     float w[6];
     fold_partials(partials, parts, w);
     if (threadIdx.x == 0) {
       s_b[0] = w[0]; s_b[1] = w[1]; s_b[2] = w[2];
       s_b[4] = w[3]; s_b[5] = w[4]; s_b[6] = w[5];
     }
-  } else if (threadIdx.x < 8) {
-    s_b[threadIdx.x] = ctl->bounds[threadIdx.x];
   }
   __syncthreads();
   float bmin[3], ext[3], rcp[3];
@@ -283,17 +279,16 @@ __global__ void k_copy_bounds(const Ctl *ctl, float *out) {
 }
 
 uint32_t launch_bounds(const float4 *tri, uint32_t n, float4 *partials,
-                       Ctl *ctl, hipStream_t s, float *cen,
-                       uint32_t fold_max) {
+                       Ctl *ctl, hipStream_t s, float *cen) {
   uint32_t blocks = (n + kMapThreads - 1) / kMapThreads;
   if (blocks > (uint32_t)kBoundsBlocks) blocks = kBoundsBlocks;
   if (blocks == 0) blocks = 1;
   hipLaunchKernelGGL(k_bounds, dim3(blocks), dim3(kMapThreads), 0, s, tri, n,
                      partials, ctl, cen);
-  if (blocks <= fold_max) return blocks;  // the consumer folds the partials
-  hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kFoldThreads), 0, s,
-                     partials, blocks, ctl);
-  return 0;
+  if (!cen)
+    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBoundsBlocks), 0, s,
+                       partials, blocks, ctl);
+  return blocks;
 }
 
 void launch_aabb_morton(const float4 *tri, uint32_t n, const MortonParams &p,
@@ -322,14 +317,14 @@ void launch_aabb_morton(const float4 *tri, uint32_t n, const MortonParams &p,
 }
 
 void launch_morton_cen(const float *cen, uint32_t n, int div_mode,
-                       uint32_t *keys, const Ctl *ctl, uint32_t *cnt, int bits,
-                       hipStream_t s, const float4 *partials, uint32_t parts) {
+                       uint32_t *keys, uint32_t *cnt, int bits, hipStream_t s,
+                       const float4 *partials, uint32_t parts) {
   const uint32_t tiles = sort_tiles(n);
   if (tiles == 0) return;
   const bool small = sort_items(n) == kSmallSortItems;
 #define LBVH_MORTON_CEN(B, T)                                              \
   hipLaunchKernelGGL((k_morton_cen<B, T>), dim3(tiles), dim3(kMapThreads), \
-                     0, s, cen, n, div_mode, keys, ctl, cnt, partials, parts)
+                     0, s, cen, n, div_mode, keys, cnt, partials, parts)
   if (bits == kWideBits) {
     if (small) LBVH_MORTON_CEN(kWideBits, kSmallSortTile);
     else LBVH_MORTON_CEN(kWideBits, kSortTile);

@@ -152,24 +152,20 @@ __global__ __launch_bounds__(kMsThreads) void k_tile_sort(
         if (tid == 0)
           for (int k = 0; k < 6; ++k) s_b[k] = v[k];
       } else {
-        // wave c folds component c, or takes the folded one
+        // wave c folds component c of the partials, kFoldPer loads in flight
         const uint32_t c = tid >> 6;
         if (c < 6) {
-          const uint32_t at = c < 3 ? c : c + 1;
-          float b = src.parts ? INFINITY : src.ctl->bounds[at];
-          if (src.parts) {
-            // the component of every partial, kFoldPer in flight per lane
-            constexpr uint32_t kFoldPer = kFoldPartialsMax / 64;
-            const float *part = reinterpret_cast<const float *>(src.partials) + at;
-            const float sign = c < 3 ? 1.f : -1.f;  // max as a min
-            float x[kFoldPer];
+          constexpr uint32_t kFoldPer = kBoundsBlocks / 64;
+          const float *part = reinterpret_cast<const float *>(src.partials) +
+                              (c < 3 ? c : c + 1);
+          const float sign = c < 3 ? 1.f : -1.f;  // max as a min
+          float x[kFoldPer], b = INFINITY;
 #pragma unroll
-            for (uint32_t q = 0; q < kFoldPer; ++q)
-              x[q] = part[8 * (size_t)min(q * 64 + (tid & 63), src.parts - 1)];
+          for (uint32_t q = 0; q < kFoldPer; ++q)
+            x[q] = part[8 * (size_t)min(q * 64 + (tid & 63), src.parts - 1)];
 #pragma unroll
-            for (uint32_t q = 0; q < kFoldPer; ++q) b = fminf(b, sign * x[q]);
-            b = sign * wave_min(b);
-          }
+          for (uint32_t q = 0; q < kFoldPer; ++q) b = fminf(b, sign * x[q]);
+          b = sign * wave_min(b);
           if ((tid & 63) == 0) s_b[c] = b;
         }
       }

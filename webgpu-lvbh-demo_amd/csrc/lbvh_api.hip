@@ -647,8 +647,8 @@ void build_radix(lbvh_ctx *ctx, const BuildScratch &S, const float4 *t4,
     StageScope sc(ctx, LBVH_STAGE_MORTON);
     uint32_t *cnt = n > 1 ? S.digits : nullptr;
     if (S.cen)
-      launch_morton_cen(S.cen, n, p.div_mode, keys, ctx->ctl, cnt, bits,
-                        ctx->stream, S.partials, parts);
+      launch_morton_cen(S.cen, n, p.div_mode, keys, cnt, bits, ctx->stream,
+                        S.partials, parts);
     else
       launch_aabb_morton(t4, n, p, from_ctl, nullptr, keys, ctx->ctl,
                          ctx->stream, cnt, bits);
@@ -668,9 +668,6 @@ void build_pipeline(lbvh_ctx *ctx, const BuildScratch &S, const float *tri,
                     uint32_t n, const float *bounds_host, void *bvh_out,
                     float *tri_out, uint32_t *sorted_keys_out,
                     int32_t *perm_out, int bits, const TreePlan &plan) {
-  // GPU bounds: the bounds pass also writes the box centres, and the Morton
-  // pass reads those (12 bytes per triangle) instead of the triangles
-  const bool use_cen = S.cen != nullptr;
   const float4 *t4 = reinterpret_cast<const float4 *>(tri);
   uint32_t *skeys = sorted_keys_out ? sorted_keys_out : S.keys_a;
   int32_t *perm = perm_out ? perm_out : S.idx_a;
@@ -678,20 +675,21 @@ void build_pipeline(lbvh_ctx *ctx, const BuildScratch &S, const float *tri,
   // a mesh of one sort tile: the tile sort takes its bounds too
   const bool whole = merge && !bounds_host && n <= (uint32_t)kMsTile;
   MortonParams p{};
-  uint32_t parts = 0;  // bounds partials the Morton pass folds itself
+  uint32_t parts = 0;  // bounds partials, folded by the kernel making the keys
   if (bounds_host) {
     p = morton_params(ctx, bounds_host);
   } else {
     p.div_mode = ctx->div_mode;
   }
   if (!bounds_host && !whole) {
+    // also writes the box centres (S.cen), which the keys are made from (12
+    // bytes per triangle instead of 48)
     StageScope sc(ctx, LBVH_STAGE_BOUNDS);
-    parts = launch_bounds(t4, n, S.partials, ctx->ctl, ctx->stream, S.cen,
-                          use_cen ? kFoldPartialsMax : 0);
+    parts = launch_bounds(t4, n, S.partials, ctx->ctl, ctx->stream, S.cen);
   }
   if (merge) {
     const MergeKeys src{nullptr, whole ? nullptr : S.cen, t4, S.partials,
-                        parts,   whole,                   ctx->ctl, p};
+                        parts,   whole,                   p};
     {
       StageScope sc(ctx, LBVH_STAGE_MORTON);
       launch_tile_sort(src, n, S.keys_b, S.idx_b, skeys, perm, S.digits,

@@ -49,7 +49,12 @@ constexpr int kTreeFrontier = 128;      // item slots per agglomeration tile
 constexpr int kItemInt4 = 3;            // 48-byte items: range, box, gap deltas
 
 constexpr int kMapThreads = 256;  // triangle-parallel kernels
-constexpr int kBoundsBlocks = 2048;  // grid of the bounds reduction
+// Grid of the bounds reduction, two blocks per CU.  So few partials are
+// folded by the kernel that makes the keys, each block for itself, which saves
+// builds a launch and the one-block fold's latency (2-5 us: 2^18 triangles
+// 71.3 -> 69.4 us, 2^20 155.8 -> 153.3, 2^22 387 -> 382); more blocks stream no
+// faster (2^24 1,319 -> 1,318 us against 2,048).
+constexpr int kBoundsBlocks = 512;
 constexpr int kMortonBlocksMax = 2048;  // grid-stride Morton (per-stage entry)
 
 // ---- device control block ------------------------------------------------
@@ -58,7 +63,7 @@ constexpr int kMortonBlocksMax = 2048;  // grid-stride Morton (per-stage entry)
 // between operations (or graph replays):
 //   fault       sticky bits (kFault*), never set in a correct run; read and
 //               cleared by lbvh_synchronize
-//   bounds      scene bounds of the last reduction (k_bounds_final)
+//   bounds      scene bounds of the last stand-alone reduction
 //   hist        global digit counts of each pass of the current sort (pass
 //               p's at hist + p * radix)
 constexpr uint32_t kFaultUpFrontier = 4u;  // per-stage up pass: a block left
@@ -90,20 +95,15 @@ struct MortonParams {
 
 // k_bounds_morton.hip
 // Scene bounds into ctl->bounds; cen (3 x cen_stride(n) floats, or null):
-// also each triangle's box centre, for launch_morton_cen.  When the reduction leaves
-// at most fold_max partials, the folding launch is skipped and the partial
-// count is returned (launch_morton_cen folds them); otherwise 0.
+// also each triangle's box centre, and the partials are left to the kernel
+// that reads the centres.  Returns their number.
 uint32_t launch_bounds(const float4 *tri, uint32_t n, float4 *partials,
-                       Ctl *ctl, hipStream_t s, float *cen = nullptr, uint32_t fold_max = 0);
+                       Ctl *ctl, hipStream_t s, float *cen = nullptr);
 // Morton keys + per-tile digit counts (as launch_aabb_morton with cnt) from
-// the centres launch_bounds wrote and the bounds in ctl, or folded from
-// `parts` bounds partials when parts != 0.
+// the centres launch_bounds wrote and its `parts` partials.
 void launch_morton_cen(const float *cen, uint32_t n, int div_mode,
-                       uint32_t *keys, const Ctl *ctl, uint32_t *cnt,
-                       int bits, hipStream_t s,
-                       const float4 *partials = nullptr, uint32_t parts = 0);
-// Bounds partials a Morton block folds itself (beyond this, k_bounds_final).
-constexpr uint32_t kFoldPartialsMax = 512;
+                       uint32_t *keys, uint32_t *cnt, int bits, hipStream_t s,
+                       const float4 *partials, uint32_t parts);
 // Box centres: x, y and z arrays of cen_stride(n) floats each (a multiple of
 // 64, so every array and every 256-triangle chunk starts 256-byte aligned
 // and is read and written 16 bytes per lane).
@@ -171,8 +171,7 @@ constexpr int kMsTile = 1 << kMsTileLog;
 constexpr uint32_t kMergeSortMax = 128u << kMsTileLog;
 // The keys of a merge sort: given (any u32; `keys` may be the output), or
 // Morton keys made by the tile sort -- from the centres launch_bounds wrote
-// with the bounds folded from `parts` partials (0: those in ctl), from the
-// triangles with the bounds in p, or (whole: n <= kMsTile) from the triangles
+// with the bounds folded from its `parts` partials, from the triangles with the bounds in p, or (whole: n <= kMsTile) from the triangles
 // with the bounds of the one tile.
 struct MergeKeys {
   const uint32_t *keys;
@@ -181,7 +180,6 @@ struct MergeKeys {
   const float4 *partials;
   uint32_t parts;
   int whole;
-  const Ctl *ctl;
   MortonParams p;
 };
 // The tile sort, then the merge rounds, both given the same buffers: the
