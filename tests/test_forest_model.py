@@ -1,12 +1,15 @@
 """The tree levels of small meshes (csrc/k_forest.hip) restated on the CPU:
 nearest smaller deltas from the waves' masks of gaps below each value, child
-boxes from a sparse table of unions, the frontier ranked by the bits of its
+boxes from the waves' sparse tables of unions, the frontier ranked by the bits of its
 first elements.  In place of the item levels' own method it must reproduce the
 oracle's nodes byte for byte."""
 import numpy as np
 import pytest
 
 import test_item_levels_model as base
+
+
+TOP = 4  # the tables' highest level
 
 
 def below_masks(deltas, m, W):
@@ -32,23 +35,42 @@ def below_masks(deltas, m, W):
 def forest_round(items, skeys, n, nodes, T=256, LOG=None):
     m = len(items)
     assert 0 < m <= T
-    W, levels = T // 64, T.bit_length() - 1
+    W = T // 64
     il, ir = [i[0] for i in items], [i[1] for i in items]
     dm = [items[0][4]] + [i[5] for i in items]
     d = dm[1:]
-    tab = [[(np.asarray(i[2], np.float32), np.asarray(i[3], np.float32)) for i in items]]
-    k = 0
-    while 2 << k < m:
-        assert k + 1 < levels
-        tab.append([(np.minimum(tab[k][t][0], tab[k][t + (1 << k)][0]),
-                     np.maximum(tab[k][t][1], tab[k][t + (1 << k)][1])) for t in range(m - (2 << k) + 1)])
-        k += 1
+    own = [(np.asarray(i[2], np.float32), np.asarray(i[3], np.float32)) for i in items]
+    union = lambda p, q: (np.minimum(p[0], q[0]), np.maximum(p[1], q[1]))  # noqa: E731
+    none = (np.full(3, np.nan, np.float32),) * 2  # past the elements: poison
+    tabs, wholes = [], []
+    for w in range(W):
+        tab = [[own[t] if t < m else none for t in range(64 * w, 64 * w + 64)]]
+        for k in range(TOP):
+            tab.append([union(tab[k][i], tab[k][i + (1 << k)]) for i in range(64 - (2 << k) + 1)])
+        tabs.append(tab)
+        whole = tab[TOP][0]
+        for i in (16, 32, 48):
+            whole = union(whole, tab[TOP][i])
+        wholes.append(whole)
+
+    def part(w, i, j):
+        k = min(TOP, (j - i + 1).bit_length() - 1)
+        # an IndexError is a read past the level
+        r = union(tabs[w][k][i], tabs[w][k][j + 1 - (1 << k)])
+        if j - i >= 2 << TOP:
+            r = union(r, union(tabs[w][TOP][i + (1 << TOP)], tabs[w][TOP][j + 1 - (2 << TOP)]))
+        return r
 
     def box(x, y):
-        k = (y - x + 1).bit_length() - 1
-        z = y + 1 - (1 << k)
-        p, q = tab[k][x], tab[k][z]  # an IndexError is a read past the table
-        return np.minimum(p[0], q[0]), np.maximum(p[1], q[1])
+        assert 0 <= x <= y < m
+        wx, wy = x >> 6, y >> 6
+        if wx == wy:
+            return part(wx, x & 63, y & 63)
+        r = union(part(wx, x & 63, 63), part(wy, 0, y & 63))
+        for w in range(wx + 1, wy):
+            r = union(r, wholes[w])
+        assert not np.isnan(r[0]).any()
+        return r
 
     masks = below_masks(d, m, W)
     span = {}
@@ -94,7 +116,7 @@ def forest_round(items, skeys, n, nodes, T=256, LOG=None):
             continue
         if (t if dm[t + 1] > dm[t] else t - 1) not in span:
             assert t not in roots
-            roots[t] = (il[t], ir[t], *tab[0][t], dm[t], dm[t + 1])
+            roots[t] = (il[t], ir[t], *own[t], dm[t], dm[t + 1])
     assert len(roots) <= base.FMAX
     return [roots[a] for a in sorted(roots)]
 

@@ -6,7 +6,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 # one tile, two; 64 and 65 leaf tiles (one item level, two); the last size
-# with direct node stores, the largest mesh and the first past it
+# with direct node stores, then past it
 SIZES = [1, 2, 63, 65, 255, 256, 257, 16384, 16385, 40001, 131072, 131073, 1 << 21, (1 << 21) + 1]
 
 
@@ -32,3 +32,20 @@ def test_build_and_refit(ctx, lb, ora, n):
         finally:
             for b in bufs:
                 b.destroy()
+
+
+@pytest.mark.parametrize("n", [300, 100000, 1 << 23, (1 << 23) + 1])
+def test_routes_agree(lb, n):
+    """Free, under a budget (which takes the larger leaf tile) and with the
+    tile fixed: the same words, up to the largest mesh and past it."""
+    side = int(np.sqrt(n / 2)) + 1
+    tri = lb.wl_heightfield(9, side, side)[:n]
+    outs = []
+    for budget, tile in [(0, 0), (64 << 30, 0), (0, 512)]:
+        with lb.Context(0, hbm_budget=budget) as c:
+            if tile:
+                c.set_tuning(lb.TUNE_TREE_TILE, tile)
+            outs.append(c.build_arrays(tri, None)[:2])
+    for bvh, otri in outs[1:]:
+        assert np.array_equal(outs[0][0], bvh)
+        assert np.array_equal(outs[0][1].view(np.uint32), otri.view(np.uint32))

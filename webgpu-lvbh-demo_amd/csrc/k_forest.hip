@@ -6,7 +6,8 @@
 //
 // A small mesh's tree is a chain of latencies.  In k_leaves most of a tile's
 // life is the climb, one dependent LDS exchange per tree level: 16,000 of
-// 25,000 cycles for a tile of 1,024 leaves.  Here a tile of kForestLeaves
+// 25,000 cycles for a tile of 1,024 leaves (11 us as a kernel; a tile here 4.5,
+// a level of items 4.5 against 8-13).  Here a tile of kForestLeaves
 // leaves (or up to kForestItems items) builds its nodes at once, a thread per
 // gap:
 //   * a gap's node spans up to the nearest gap with a smaller delta on either
@@ -14,9 +15,10 @@
 //     delta is below u, built from the deltas' six bit planes; a gap of delta
 //     v reads the masks of v, its own wave's first, and the nearest set bits
 //     are its bounds;
-//   * the boxes of the node's two children are range unions: a sparse table
-//     of unions of 2^k elements answers each with two reads.  It takes 24
-//     bytes per element and level, which is why the tiles are small;
+//   * the boxes of the node's two children are range unions: a wave's sparse
+//     table of unions of 2^k elements answers each with two reads (or a few,
+//     across waves).  It takes 24 bytes per entry, which is why the tiles are
+//     small;
 //   * nodes and elements whose parent gap has no node in the tile are its
 //     frontier, ranked by the bits of their first elements.
 #include "tree_util.h"
@@ -26,18 +28,30 @@ namespace lbvh {
 constexpr int kForestLeaves = kForestTile;
 constexpr int kForestItems = 512;
 
+// A wave's sparse table: entry i of level k is the union of its elements [i, i
+// + 2^k), for k <= kTop and those i whose range ends in the wave.  A level
+// less than the wave needs (ranges past 2^(kTop + 1) take two lookups more)
+// lets five leaf tiles share a CU's LDS, not four.
+constexpr int kTop = 4;
+__host__ __device__ constexpr int table_level(int k) { return 65 * k - (1 << k) + 1; }
+constexpr int kTable = table_level(kTop + 1);
+
 template <int T>
 struct ForestLds {
-  static constexpr int kLevels = T == 256 ? 8 : 9;  // ranges of up to T - 1
-  static_assert(1 << kLevels == T, "sparse table levels");
-  float4 a[kLevels][T];  // min.xyz, max.x of the union of 2^k elements
-  float2 b[kLevels][T];  // max.yz
+  float4 a[T / 64][kTable + 1];  // min.xyz, max.x; the last one: the whole wave
+  float2 b[T / 64][kTable + 1];  // max.yz
   uint64_t below[T / 64][64];  // [wave][u]: its gaps with a delta below u
   uint64_t node_bits[T / 64];  // gaps whose node is complete in the tile
   uint64_t root_bits[T / 64];  // first elements of the frontier
   uint64_t id_bits[T / 64];    // node ids made here (kStage)
   signed char dm[T + 4];       // deltas by position: dm[p] before element p
 };
+
+// LDS written by a wave for itself: its operations complete in issue order.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 
 // Lanes whose value is below v, from the values' bit planes (as k_rt_tiles).
 __device__ __forceinline__ uint64_t planes_below(const uint64_t (&pl)[6],
@@ -52,16 +66,54 @@ __device__ __forceinline__ uint64_t planes_below(const uint64_t (&pl)[6],
   return lt;
 }
 
+struct Box {
+  float mn[3], mx[3];
+};
+template <int T>
+__device__ __forceinline__ void join(const ForestLds<T> &L, int w, int e, Box &x) {
+  const float4 p = L.a[w][e];
+  const float2 r = L.b[w][e];
+  x.mn[0] = qmin(x.mn[0], p.x); x.mn[1] = qmin(x.mn[1], p.y);
+  x.mn[2] = qmin(x.mn[2], p.z); x.mx[0] = qmax(x.mx[0], p.w);
+  x.mx[1] = qmax(x.mx[1], r.x); x.mx[2] = qmax(x.mx[2], r.y);
+}
+template <int T>
+__device__ __forceinline__ Box entry(const ForestLds<T> &L, int w, int e) {
+  const float4 p = L.a[w][e];
+  const float2 r = L.b[w][e];
+  return {{p.x, p.y, p.z}, {p.w, r.x, r.y}};
+}
+
+// Joins wave w's elements [i, j] to x, entry i of the level that halves the
+// range already in it.
+__device__ __forceinline__ int range_level(int i, int j) {
+  return min(kTop, 31 - __clz(j - i + 1));
+}
+template <int T>
+__device__ __forceinline__ void join_rest(const ForestLds<T> &L, int w, int i,
+                                          int j, int k, Box &x) {
+  join(L, w, table_level(k) + j + 1 - (1 << k), x);
+  if (j - i >= 2 << kTop) {
+    join(L, w, table_level(kTop) + i + (1 << kTop), x);
+    join(L, w, table_level(kTop) + j + 1 - (2 << kTop), x);
+  }
+}
+
 // Union of elements [x, y].
 template <int T>
-__device__ __forceinline__ void forest_box(const ForestLds<T> &L, int x, int y,
-                                           float mn[3], float mx[3]) {
-  const int k = 31 - __clz(y - x + 1);
-  const int z = y + 1 - (1 << k);
-  const float4 p = L.a[k][x], q = L.a[k][z];
-  const float2 r = L.b[k][x], s = L.b[k][z];
-  mn[0] = qmin(p.x, q.x); mn[1] = qmin(p.y, q.y); mn[2] = qmin(p.z, q.z);
-  mx[0] = qmax(p.w, q.w); mx[1] = qmax(r.x, s.x); mx[2] = qmax(r.y, s.y);
+__device__ __forceinline__ Box forest_box(const ForestLds<T> &L, int x, int y) {
+  const int wx = x >> 6, wy = y >> 6;
+  const int i = x & 63, j = wx == wy ? y & 63 : 63;
+  const int k = range_level(i, j);
+  Box r = entry(L, wx, table_level(k) + i);
+  join_rest(L, wx, i, j, k, r);
+  if (wx != wy) {
+    const int t = y & 63, kt = range_level(0, t);
+    join(L, wy, table_level(kt), r);
+    join_rest(L, wy, 0, t, kt, r);
+    for (int w = wx + 1; w < wy; ++w) join(L, w, kTable, r);
+  }
+  return r;
 }
 
 // The forest over m <= T elements.  Thread tid < m passes element tid: its
@@ -87,8 +139,6 @@ __device__ __forceinline__ ForestRoot forest_round(
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool elem = tid < m;
-  L.a[0][tid] = make_float4(mn[0], mn[1], mn[2], mx[0]);
-  L.b[0][tid] = make_float2(mx[1], mx[2]);
   if (elem) L.dm[tid + 1] = (signed char)d;
   if (tid == 0) L.dm[0] = (signed char)d0;
   {
@@ -101,46 +151,48 @@ __device__ __forceinline__ ForestRoot forest_round(
     L.below[w][lane] = planes_below(pl, lane) | ends;
   }
   if (tid < W) L.root_bits[tid] = L.id_bits[tid] = 0ull;
-  __syncthreads();
-  // the gap after element tid, its masks read while the table is built
-  const bool gap = tid < m - 1;
-  uint64_t mask[W];
-#pragma unroll
-  for (int q = 0; q < W; ++q) mask[q] = L.below[q][gap ? d : 0];
   {
-    float4 p = L.a[0][tid];
-    float2 r = L.b[0][tid];
-    for (int k = 0; 2 << k < m; ++k) {  // ranges of fewer than m elements
-      const int o = tid + (1 << k);
-      if (tid + (2 << k) <= m) {
-        const float4 q = L.a[k][o];
-        const float2 s = L.b[k][o];
-        p = make_float4(qmin(p.x, q.x), qmin(p.y, q.y), qmin(p.z, q.z),
-                        qmax(p.w, q.w));
-        r = make_float2(qmax(r.x, s.x), qmax(r.y, s.y));
-        L.a[k + 1][tid] = p;
-        L.b[k + 1][tid] = r;
-      }
-      __syncthreads();
+    Box x = {{mn[0], mn[1], mn[2]}, {mx[0], mx[1], mx[2]}};
+    const auto put = [&](int e) {
+      L.a[w][e] = make_float4(x.mn[0], x.mn[1], x.mn[2], x.mx[0]);
+      L.b[w][e] = make_float2(x.mx[1], x.mx[2]);
+      wave_lds_fence();
+    };
+    put(lane);
+#pragma unroll
+    for (int k = 0; k < kTop; ++k) {
+      // lanes past the level repeat its last entry
+      const int i = min(lane, 64 - (2 << k));
+      x = entry(L, w, table_level(k) + i);
+      join(L, w, table_level(k) + i + (1 << k), x);
+      put(table_level(k + 1) + i);
     }
+    join(L, w, table_level(kTop) + 16, x);  // lane 0: the whole wave
+    join(L, w, table_level(kTop) + 32, x);
+    join(L, w, table_level(kTop) + 48, x);
+    if (lane == 0) put(kTable);
   }
-  // nearest smaller deltas: positions pl and pr (-1: none in the tile)
+  __syncthreads();
+  // nearest smaller deltas: positions pl and pr (-1: none in the tile); the
+  // gap after element 64 q + bit is position 64 q + bit + 1
+  const bool gap = tid < m - 1;
   int pl = -1, pr = -1;
   if (gap) {
-#pragma unroll
-    for (int q = 0; q < W; ++q) {
-      uint64_t lo = mask[q], hi = mask[q];
-      if (q == w) {
-        lo &= (1ull << lane) - 1;
-        hi &= lane == 63 ? 0ull : ~((2ull << lane) - 1);
-      }
-      // gaps after element 64 q + bit are positions 64 q + bit + 1
-      if (q <= w && lo) pl = q * 64 + 64 - (int)__clzll((long long)lo);
-      if (q >= w && hi && pr < 0)
-        pr = q * 64 + (int)__ffsll((unsigned long long)hi);
-    }
-    if (pl < 0 && L.dm[0] < d) pl = 0;
+    const uint64_t mask = L.below[w][d];
+    const uint64_t lo = mask & ((1ull << lane) - 1);
+    const uint64_t hi = lane == 63 ? 0ull : mask & ~((2ull << lane) - 1);
+    if (lo) pl = w * 64 + 64 - (int)__clzll((long long)lo);
+    if (hi) pr = w * 64 + (int)__ffsll((unsigned long long)hi);
   }
+  for (int q = w - 1; q >= 0 && __ballot(gap && pl < 0); --q) {
+    const uint64_t mask = L.below[q][gap ? d : 0];
+    if (gap && pl < 0 && mask) pl = q * 64 + 64 - (int)__clzll((long long)mask);
+  }
+  for (int q = w + 1; q * 64 < m && __ballot(gap && pr < 0); ++q) {
+    const uint64_t mask = L.below[q][gap ? d : 0];
+    if (gap && pr < 0 && mask) pr = q * 64 + (int)__ffsll((unsigned long long)mask);
+  }
+  if (gap && pl < 0 && L.dm[0] < d) pl = 0;
   const bool node = pl >= 0 && pr >= 0;
   const uint64_t made = __ballot(node);
   if (lane == 0) L.node_bits[w] = made;
@@ -155,16 +207,14 @@ __device__ __forceinline__ ForestRoot forest_round(
   if (node) {
     const int x = pl, y = pr - 1;
     const int dl = L.dm[pl], dr = L.dm[pr];
-    float lmn[3], lmx[3], rmn[3], rmx[3];
-    forest_box(L, x, tid, lmn, lmx);
-    forest_box(L, tid + 1, y, rmn, rmx);
+    const Box lb = forest_box(L, x, tid), rb = forest_box(L, tid + 1, y);
     const int lo = range(x).x, s = range(tid).y, hi = range(y).y;
     const bool whole = lo == 0 && hi == N - 1;
     const int K = whole ? 0 : (dr > dl ? hi : lo);
-    quad[0] = pack3(lmn, lo == s ? -(s + 1) : s);
-    quad[1] = pack3(lmx, 2);
-    quad[2] = pack3(rmn, hi == s + 1 ? -(s + 2) : s + 1);
-    quad[3] = pack3(rmx, 0);
+    quad[0] = pack3(lb.mn, lo == s ? -(s + 1) : s);
+    quad[1] = pack3(lb.mx, 2);
+    quad[2] = pack3(rb.mn, hi == s + 1 ? -(s + 2) : s + 1);
+    quad[3] = pack3(rb.mx, 0);
     slot = K - ts;
     if (kStage) {
       atomicOr(reinterpret_cast<unsigned long long *>(&L.id_bits[slot >> 6]),
@@ -179,8 +229,8 @@ __device__ __forceinline__ ForestRoot forest_round(
       R.l = lo; R.r = hi; R.dl = dl; R.dr = dr;
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
-        R.mn[c] = qmin(lmn[c], rmn[c]);
-        R.mx[c] = qmax(lmx[c], rmx[c]);
+        R.mn[c] = qmin(lb.mn[c], rb.mn[c]);
+        R.mx[c] = qmax(lb.mx[c], rb.mx[c]);
       }
     }
   }
@@ -216,6 +266,7 @@ __device__ __forceinline__ ForestRoot forest_round(
   if (kStage) {
     // a leaf tile's node ids are its own positions: in id order through LDS
     // (the table is no longer read), four lanes per 64-byte node
+    static_assert(!kStage || 4 * T <= W * (kTable + 1), "a quad per node");
     int4 *stage = reinterpret_cast<int4 *>(&L.a[0][0]);
     if (node) {
 #pragma unroll
@@ -253,8 +304,8 @@ __device__ __forceinline__ void forest_emit(const ForestRoot &R, uint32_t tile,
 // boxes as k_leaves does.  kStage: the nodes go out in id order through LDS,
 // four lanes per node; a mesh of at most kForestDirect leaves, whose tiles are
 // latency alone, stores them from the threads that made them (a build of 1,500
-// 20.4 -> 19.7 us; one of 2^18 71.1 against 71.9 us staged, of 2^22 380
-// against 412).
+// 20.4 -> 19.7 us; one of 2^18 71.9 against 71.1 us staged, of 2^22 412
+// against 380).
 constexpr uint32_t kForestDirect = 1u << 17;
 template <bool kStage>
 __global__ __launch_bounds__(kForestLeaves) void k_forest_leaves(
@@ -271,9 +322,10 @@ __global__ __launch_bounds__(kForestLeaves) void k_forest_leaves(
   const uint32_t k = (uint32_t)ts + tid;
   float mn[3] = {0.f, 0.f, 0.f}, mx[3] = {0.f, 0.f, 0.f};
   int d = -1, d0 = -1;
-  // O_TRI goes out through LDS, in table levels that are built later
-  static_assert(3 * sizeof(int4) <= 3 * sizeof(L.a[0][0]), "three levels");
-  int4 *stage = reinterpret_cast<int4 *>(&L.a[ForestLds<T>::kLevels - 3][0]);
+  // O_TRI goes out through LDS, each wave's 192 int4s through its own table
+  static_assert(3 * 64 <= kTable, "a wave's triangles");
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  int4 *stage = reinterpret_cast<int4 *>(&L.a[w][0]);
   if (tid < m) {
     const uint32_t pi = (uint32_t)perm[k];
     const uint32_t k_here = skeys[k];
@@ -281,9 +333,9 @@ __global__ __launch_bounds__(kForestLeaves) void k_forest_leaves(
     const uint32_t k_0 = skeys[ts], k_prev = skeys[ts > 0 ? ts - 1 : 0];
     const size_t src = 3 * (size_t)(pi < N ? pi : 0u);
     const int4 a = tri[src], b = tri[src + 1], c = tri[src + 2];
-    stage[3 * tid] = a;
-    stage[3 * tid + 1] = b;
-    stage[3 * tid + 2] = c;
+    stage[3 * lane] = a;
+    stage[3 * lane + 1] = b;
+    stage[3 * lane + 2] = c;
     tri_box(a, b, c, mn, mx);
     perturb(mn, mx);
     const int d_next = delta_next(k_here, k_next, k);
@@ -291,15 +343,16 @@ __global__ __launch_bounds__(kForestLeaves) void k_forest_leaves(
     d = k + 1 < N ? d_next : -1;
     d0 = ts > 0 ? d_prev : -1;
   }
-  __syncthreads();
+  wave_lds_fence();
   {
-    int4 *o = otri + 3 * (size_t)ts;
+    int4 *o = otri + 3 * (size_t)(ts + 64 * w);
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-      const int e = j * T + tid;
-      if (e < 3 * m) store_nt(o + e, stage[e]);
+      const int e = j * 64 + lane;
+      if (e < 3 * (m - 64 * w)) store_nt(o + e, stage[e]);
     }
   }
+  wave_lds_fence();  // the table is written next
   if (N == 1) {
     if (tid == 0) {
       write_single_leaf_node(nodes, mn, mx);

@@ -459,14 +459,20 @@ int untuned_bits(uint32_t n) {
 }
 
 // The tree levels of an n-triangle mesh: leaf tile, and whether they are
-// k_forest.hip's (small meshes, unless the tile is fixed).
+// k_forest.hip's: meshes of at most kForestMax triangles, unless the tile is
+// fixed.  Small tiles want four times the item slots of the default ones (25
+// bytes a triangle against 6), so a context with an HBM budget keeps to its
+// larger tile: what fitted the budget still does.
 struct TreePlan {
   int tile;
   bool forest;
 };
 TreePlan tree_plan(const lbvh_ctx *ctx, uint32_t n) {
-  if (n <= kForestMax && !ctx->tree_tile_fixed) return {kForestTile, true};
-  return {tile_for(ctx, n), false};
+  const int tile = tile_for(ctx, n);
+  const bool room = ctx->budget == 0 || tile == kForestTile;
+  if (n <= kForestMax && !ctx->tree_tile_fixed && room)
+    return {kForestTile, true};
+  return {tile, false};
 }
 
 int bits_for(const lbvh_ctx *ctx, uint32_t n) {

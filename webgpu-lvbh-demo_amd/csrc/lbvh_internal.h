@@ -241,12 +241,12 @@ void launch_tree_level(int level, int tile, uint32_t grid, const float4 *tri,
 // k_forest.hip
 // One agglomeration level of a mesh of at most kForestMax leaves, over leaf
 // tiles of kForestTile: the arguments, items and level plan of
-// launch_tree_level.  Refits (this against the best leaf tile there): 1,500
-// leaves 9.7 / 17.3 us, 2^16 17.3 / 24.5, 2^18 28 / 37, 2^20 66 / 72, 2^21 109 /
-// 117 uniform and 89 / 92 on a heightfield; at 2^22 the heightfield turns (192
-// / 161), where k_leaves keeps 2,048 leaves per CU in flight against 768 here.
+// launch_tree_level.  Refits, this against the best leaf tile of k_leaves:
+// 1,500 leaves 9.4 / 17.3 us, 2^16 16.3 / 24.5, 2^18 24.7 / 37, 2^20 63 / 72
+// (uniform) and 48 / 59 (heightfield), 8M 368 / 380 and 287 / 293; at 2^24 it
+// turns (838 / 798, 577 / 555).
 constexpr int kForestTile = 256;
-constexpr uint32_t kForestMax = 1u << 21;
+constexpr uint32_t kForestMax = 1u << 23;
 void launch_forest_level(int level, uint32_t grid, const float4 *tri,
                          const uint32_t *skeys, const int32_t *perm,
                          uint32_t n, float4 *otri, const int4 *items_in,
