@@ -43,7 +43,8 @@ namespace lbvh {
 // are numbered g and g + 1 (leaves when single), so gap g writes exactly the
 // parents slots g or n + g, and g + 1 or n + g + 1 (radix-tree.js:146-156).
 //
-// Three launches, no waiting between blocks:
+// Three launches (two for few tiles, k_rt_resolve_few), no waiting between
+// blocks:
 //   k_rt_tiles    a block takes 4,096 gaps: deltas from its keys in LDS, L
 //                 and R inside 64-gap segments from bit-plane ballots, then
 //                 across the tile's segments from per-segment tables of the
@@ -59,8 +60,10 @@ namespace lbvh {
 //                 each tile: a prefix max (suffix min) over tiles.
 //   k_rt_resolve  each record takes its missing bound from the scans and
 //                 writes its slots.
-constexpr int kRtThreads = 256;
-constexpr int kRtPer = 16;                          // gaps per thread
+// 16 waves per tile: with 4, a small mesh's few tiles were one long chain (the
+// stage 22.5 us at 3,000 leaves, now 14; 3M leaves 35.5 and 29.5).
+constexpr int kRtThreads = 1024;
+constexpr int kRtPer = 4;                           // gaps per thread
 constexpr int kRtTile = kRtThreads * kRtPer;        // 4096 gaps per tile
 constexpr int kRtSegs = kRtTile / 64;               // 64-gap segments
 constexpr int kRtRecords = 128;                     // spine gaps per tile
@@ -303,6 +306,63 @@ __global__ __launch_bounds__(kRtScanThreads) void k_rt_scan(
   }
 }
 
+// Writes a record's slots, the bounds that its tile lacks from the summaries
+// before and after the tile (none: the sentinels).
+__device__ __forceinline__ void rt_finish(int32_t *__restrict__ par, uint32_t n,
+                                          const int4 &rec,
+                                          unsigned long long before,
+                                          unsigned long long after) {
+  const int flags = (rec.y >> 8) & 3;
+  int dL = ((rec.y >> 16) & 0xFF) - 1, dR = ((rec.y >> 24) & 0xFF) - 1;
+  int64_t L = rec.z, R = rec.w;
+  if (flags & 1) {
+    L = before ? (int64_t)(before >> 8) - 1 : -1;
+    dL = before ? (int)(before & 0xFF) : -1;
+  }
+  if (flags & 2) {
+    R = after != ~0ull ? (int64_t)(after >> 8) : (int64_t)n - 1;
+    dR = after != ~0ull ? (int)(after & 0xFF) : -1;
+  }
+  rt_write(par, n, rec.x, L, dL, R, dR);
+}
+
+// The spine gaps of at most kRtFewTiles tiles: k_rt_resolve without a scan
+// before it.  Sixteen lanes take a record and look through the summaries of
+// the tiles before and after for themselves, four loads a lane in flight (the
+// stage 14 -> 10.5 us at 3,000 leaves, 15.7 -> 12.3 at 60,000); the loads grow
+// with the tiles, a launch does not.
+constexpr int kRtFewTiles = 64;
+constexpr int kRtFewThreads = 1024;
+__global__ __launch_bounds__(kRtFewThreads) void k_rt_resolve_few(
+    int32_t *__restrict__ par, uint32_t n, const int4 *__restrict__ recs,
+    const uint32_t *__restrict__ rec_cnt,
+    const unsigned long long *__restrict__ last,
+    const unsigned long long *__restrict__ first, uint32_t tiles) {
+  const uint32_t t = blockIdx.x;
+  const int sub = threadIdx.x & 15;
+  const uint32_t cnt = min(rec_cnt[t], (uint32_t)kRtRecords);
+  for (uint32_t r = threadIdx.x >> 4; r < cnt; r += kRtFewThreads / 16) {
+    const int4 rec = recs[(size_t)t * kRtRecords + r];
+    const int v = rec.y & 63;
+    unsigned long long before = 0ull, after = ~0ull;
+#pragma unroll
+    for (int k = 0; k < kRtFewTiles; k += 16) {
+      const uint32_t q = (uint32_t)(k + sub);
+      if (q >= tiles) continue;
+      const unsigned long long a = last[(size_t)v * tiles + q];
+      const unsigned long long b = first[(size_t)v * tiles + q];
+      if (q < t) before = max(before, a);
+      if (q > t) after = min(after, b);
+    }
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) {
+      before = max(before, __shfl_xor(before, o, 16));
+      after = min(after, __shfl_xor(after, o, 16));
+    }
+    if (sub == 0) rt_finish(par, n, rec, before, after);
+  }
+}
+
 // The spine gaps: missing bounds from the scans (none: the sentinels).
 __global__ __launch_bounds__(kRtRecords) void k_rt_resolve(
     int32_t *__restrict__ par, uint32_t n, const int4 *__restrict__ recs,
@@ -311,31 +371,9 @@ __global__ __launch_bounds__(kRtRecords) void k_rt_resolve(
     const unsigned long long *__restrict__ first, uint32_t tiles) {
   const uint32_t t = blockIdx.x;
   if (threadIdx.x >= rec_cnt[t]) return;
-  const int4 r = recs[(size_t)t * kRtRecords + threadIdx.x];
-  const int v = r.y & 0xFF, flags = (r.y >> 8) & 3;
-  int dL = ((r.y >> 16) & 0xFF) - 1, dR = ((r.y >> 24) & 0xFF) - 1;
-  int64_t L = r.z, R = r.w;
-  if (flags & 1) {
-    const unsigned long long e = last[(size_t)v * tiles + t];
-    if (e == 0ull) {
-      L = -1;
-      dL = -1;
-    } else {
-      L = (int64_t)(e >> 8) - 1;
-      dL = (int)(e & 0xFF);
-    }
-  }
-  if (flags & 2) {
-    const unsigned long long e = first[(size_t)v * tiles + t];
-    if (e == ~0ull) {
-      R = (int64_t)n - 1;
-      dR = -1;
-    } else {
-      R = (int64_t)(e >> 8);
-      dR = (int)(e & 0xFF);
-    }
-  }
-  rt_write(par, n, r.x, L, dL, R, dR);
+  const int4 rec = recs[(size_t)t * kRtRecords + threadIdx.x];
+  const int v = rec.y & 63;
+  rt_finish(par, n, rec, last[(size_t)v * tiles + t], first[(size_t)v * tiles + t]);
 }
 
 // ---------------------------------------------------------------------------
@@ -354,13 +392,14 @@ __global__ __launch_bounds__(kRtRecords) void k_rt_resolve(
 // completes on chip.  The subtrees that cannot complete there -- the
 // block's maximal complete subtrees, at most two per level of the tree, so
 // at most kUpFront -- leave as items, in leaf order, for k_up_items, which
-// merges the items of kUpFanIn neighbouring blocks the same way, level
+// merges the items of a fixed number of neighbouring blocks the same way, level
 // after level, until one block holds the root.  No block ever waits for
 // another: kernel boundaries order the levels.
 constexpr int kUpTile = 1024;
 constexpr int kUpFront = 128;  // items a block leaves at most (2 per level)
-constexpr int kUpFanIn = 32;   // blocks of the level below per item block
-static_assert(kUpFanIn < kUpTile && kUpFront < kUpTile,
+constexpr int kUpFanIn = 32;   // blocks of the level below per item block,
+constexpr int kUpFanInMax = 64;  // or this many (up_levels)
+static_assert(kUpFanInMax < kUpTile && kUpFront < kUpTile,
               "one thread per source block; a round takes new items");
 
 struct UpLds {
@@ -373,37 +412,21 @@ struct UpLds {
   int32_t far[2][kUpTile];
   // the block's parents entries, ids ts .. te (one past the block, for the
   // sibling test at its edge): a climb reads these at every step, and from
-  // global memory they made each step a chain of dependent loads
+  // global memory they made each step a chain of dependent loads.  First as
+  // they are, then as links (up_link_of).
   int32_t par_leaf[kUpTile + 1];  // parents[n + id]
   int32_t par_node[kUpTile + 1];  // parents[id]
 };
 
-// parents[n + id] / parents[id] for id in the block's staged range
-// [ts, ts + kUpTile].  A climb only asks for ids there: it climbs through
-// leaves and nodes of the block's range [ts, te) and reads their successor
-// (<= te) and, for a node inside the range, its parent entry.  The index is
-// clamped all the same, and the arrays are read from LDS only: a choice
-// between LDS and global memory per lane compiles to a generic (flat) load,
-// which waits on the vector memory path at every step of the climb.
-__device__ __forceinline__ int32_t up_par_leaf(const UpLds &L, int32_t ts,
-                                               int32_t id) {
-  const int32_t k = id - ts;
-  return L.par_leaf[k < 0 ? 0 : (k > kUpTile ? kUpTile : k)];
-}
-__device__ __forceinline__ int32_t up_par_node(const UpLds &L, int32_t ts,
-                                               int32_t id) {
-  const int32_t k = id - ts;
-  return L.par_node[k < 0 ? 0 : (k > kUpTile ? kUpTile : k)];
-}
-
-// Node num (a leaf when leaf) is its parent p's left child when the child
-// numbered one above it has the same parent.
-__device__ __forceinline__ bool up_is_left(const UpLds &L, uint32_t n,
-                                           int32_t ts, int32_t num,
-                                           int32_t p) {
-  const int32_t sib = num + 1;
-  return (sib <= (int32_t)n - 1 && up_par_leaf(L, ts, sib) == p) ||
-         (sib <= (int32_t)n - 2 && up_par_node(L, ts, sib) == p);
+// The link of a node to its parent p: 2 p + side (p < 2^30), kUpNoLink where p
+// is no node.  A child is its parent's left one when the child numbered one above it
+// (leaf_sib, node_sib: that number's entries) has the same parent.
+constexpr int32_t kUpNoLink = -1;
+__device__ __forceinline__ int32_t up_link_of(int32_t p, uint32_t n,
+                                              int32_t leaf_sib,
+                                              int32_t node_sib) {
+  if (p < 0 || p >= (int32_t)n - 1) return kUpNoLink;
+  return 2 * p + (leaf_sib == p || node_sib == p ? 0 : 1);
 }
 
 // An item: a complete subtree that has still to arrive at its parent.
@@ -517,13 +540,20 @@ __global__ __launch_bounds__(kUpTile) void k_up_pass(
     mx[1] = __builtin_canonicalizef(__int_as_float(bh.y));
     mx[2] = __builtin_canonicalizef(__int_as_float(bh.z));
   }
+  // (-1, no node, also past the last leaf n - 1 and the last node n - 2)
   L.cnt[tid] = 0u;
   L.par_leaf[tid] = in ? pl : -1;
-  L.par_node[tid] = in ? pn : -1;
+  L.par_node[tid] = g < (int64_t)n - 1 ? pn : -1;
   if (tid == 0) {
     L.par_leaf[kUpTile] = in_e ? pl_e : -1;
-    L.par_node[kUpTile] = in_e ? pn_e : -1;
+    L.par_node[kUpTile] = e < (int64_t)n - 1 ? pn_e : -1;
   }
+  __syncthreads();
+  const int32_t leaf_sib = L.par_leaf[tid + 1], node_sib = L.par_node[tid + 1];
+  const int32_t leaf_link = up_link_of(L.par_leaf[tid], n, leaf_sib, node_sib);
+  const int32_t node_link = up_link_of(L.par_node[tid], n, leaf_sib, node_sib);
+  __syncthreads();
+  L.par_node[tid] = node_link;  // read by the climbs
   __syncthreads();
   // 0: done, 1: first to arrive at a parent in LDS, 2: pending (an item)
   int mode = 0;
@@ -543,13 +573,14 @@ __global__ __launch_bounds__(kUpTile) void k_up_pass(
         int4 *lastn = nodes + 4 * (size_t)(n - 1);
         lastn[0] = z; lastn[1] = z; lastn[2] = z; lastn[3] = z;
       }
-      p = L.par_leaf[tid];
+      int32_t link = leaf_link;
       // A valid tree is at most 64 levels deep (each level consumes a bit of
       // the 62-bit position-augmented key); the step cap and the range
       // check keep a malformed parents array from running away.
       for (int step = 0; step < 128; ++step) {
-        if (p < 0 || p >= (int32_t)n - 1) break;
-        side = up_is_left(L, n, (int32_t)ts, (int32_t)num, p) ? 0 : 1;
+        if (link == kUpNoLink) break;
+        p = link >> 1;
+        side = link & 1;
         self = leaf ? -(int)(num + 1) : (int)num;
         if (p < ts || p >= te) {  // the parent lies outside the block
           mode = 2;
@@ -579,7 +610,7 @@ __global__ __launch_bounds__(kUpTile) void k_up_pass(
         if (p == 0) break;  // root merged
         leaf = false;
         num = p;
-        p = up_par_node(L, (int32_t)ts, p);
+        link = L.par_node[slot];
       }
     }
   }
@@ -618,8 +649,20 @@ __global__ __launch_bounds__(kUpTile) void k_up_pass(
           self, lo, hi, p, side, mn, mx);
 }
 
-// One level of items: block b takes the items of blocks [kUpFanIn b,
-// kUpFanIn b + kUpFanIn) of the level below, in leaf order.  Those items
+// Counts an arrival at a counter in LDS, ordered with the block's other LDS
+// accesses only.  A plain acq_rel operation also waits for the wave's stores
+// to global memory (here the node halves), once per step of a climb (the pass
+// 160 -> 154.5 us at 3M leaves, 315 -> 296 at 8M).
+__device__ __forceinline__ uint32_t lds_arrive(uint32_t *cnt) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  const uint32_t old = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_WORKGROUP);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  return old;
+}
+
+// One level of items: block b takes the items of blocks [fan b, fan b + fan)
+// of the level below, in leaf order.  Those items
 // partition a leaf range, and the split of every node still to complete
 // inside it is a gap between two adjacent items: arrivals meet in that
 // gap's LDS slot (the left child at the gap after its last item, the right
@@ -640,12 +683,32 @@ struct UpItemLds {
   int32_t far_leaf[2][kUpTile];  // [side][gap]: far leaf
   uint32_t cnt[kUpTile];      // arrivals per gap
   uint32_t mark[kUpTile];     // item ordering
-  uint32_t base[kUpFanIn + 1];  // first item of each source block
+  // [gap]: the node that splits there and its own parent and side, as a tree
+  // has them.  A climb that read them from the parents array at each step
+  // was a chain of dependent global loads (the pass 172 us at 3M leaves, with
+  // these 160).
+  int32_t node[kUpTile];
+  int32_t node_par[kUpTile];
+  uint8_t node_side[kUpTile];
+  uint32_t base[kUpFanInMax + 1];  // first item of each source block
 };
+
+// Node num's parent, and its side there.
+struct UpLink {
+  int32_t p;
+  int side;
+};
+__device__ __forceinline__ UpLink up_link(const int32_t *__restrict__ par,
+                                          uint32_t n, int32_t num) {
+  const int32_t pl = num + 1 <= (int32_t)n - 1 ? par[n + num + 1] : -2;
+  const int32_t pn = num + 1 <= (int32_t)n - 2 ? par[num + 1] : -2;
+  const int32_t p = par[num];
+  return {p, (pl == p || pn == p) ? 0 : 1};
+}
 
 __global__ __launch_bounds__(kUpTile) void k_up_items(
     const int4 *__restrict__ items_in, const uint32_t *__restrict__ cnt_in,
-    const uint32_t *__restrict__ done_in, uint32_t tiles_in,
+    const uint32_t *__restrict__ done_in, uint32_t tiles_in, uint32_t fan,
     int4 *items_out,  // written, then read back by the next round
     uint32_t *__restrict__ cnt_out, uint32_t *__restrict__ done_out,
     const int32_t *__restrict__ par, uint32_t n, int4 *nodes, Ctl *ctl,
@@ -655,20 +718,20 @@ __global__ __launch_bounds__(kUpTile) void k_up_items(
   __shared__ uint32_t s_done;
   const int tid = threadIdx.x;
   const uint32_t tile = blockIdx.x;
-  const uint32_t c0 = tile * kUpFanIn;
-  const uint32_t nc = min((uint32_t)kUpFanIn, tiles_in - c0);
+  const uint32_t c0 = tile * fan;
+  const uint32_t nc = min(fan, tiles_in - c0);
   {
     const uint32_t c =
         (uint32_t)tid < nc ? min(cnt_in[c0 + tid], (uint32_t)kUpFront) : 0u;
     const uint32_t ex = block_exclusive_scan(c, s_wsum);
-    if (tid <= kUpFanIn) S.base[tid] = ex;  // the total from nc on
+    if (tid <= kUpFanInMax) S.base[tid] = ex;  // the total from nc on
   }
   // nodes completed by the source blocks, then by each round here: the last
   // level holds the count of the whole tree
   uint32_t completed = (uint32_t)tid < nc ? done_in[c0 + tid] : 0u;
   int4 *own = items_out + 3 * (size_t)tile * kUpFront;
   __syncthreads();
-  const int total = (int)S.base[kUpFanIn];
+  const int total = (int)S.base[kUpFanInMax];
   int taken = 0;  // source items used by earlier rounds
   int carry = 0;  // items left pending by the previous round
   while (true) {
@@ -691,7 +754,7 @@ __global__ __launch_bounds__(kUpTile) void k_up_items(
         const uint32_t g = (uint32_t)(taken + tid - carry);
         uint32_t j = 0;
 #pragma unroll
-        for (uint32_t step = kUpFanIn / 2; step > 0; step >>= 1)
+        for (uint32_t step = kUpFanInMax / 2; step > 0; step >>= 1)
           if (j + step < nc && S.base[j + step] <= g) j += step;
         it = items_in + 3 * ((size_t)(c0 + j) * kUpFront + (g - S.base[j]));
       }
@@ -702,6 +765,21 @@ __global__ __launch_bounds__(kUpTile) void k_up_items(
       mx[0] = __int_as_float(c.x); mx[1] = __int_as_float(c.y);
       mx[2] = __int_as_float(c.z);
       mode = 2;
+      // The split's children are numbered hi and hi + 1 and share a parent,
+      // the node.  Input that is no tree may give another one: the climb asks
+      // the array where its parent is not this node.
+      const int32_t h = hi < 0 || hi >= (int32_t)n - 1 ? 0 : hi;  // n >= 2
+      const int32_t a0 = par[n + h], a1 = par[h], b0 = par[n + h + 1];
+      const int32_t b1 = h + 1 <= (int32_t)n - 2 ? par[h + 1] : -2;
+      const int32_t node_id = a0 == b0 || a0 == b1 ? a0 : a1;
+      const int32_t num = node_id < 0 || node_id >= (int32_t)n - 1 ? 0 : node_id;
+      const UpLink up = up_link(par, n, num);
+      S.node[tid] = node_id == num ? num : -1;
+      S.node_par[tid] = up.p;
+      S.node_side[tid] = (uint8_t)up.side;
+    }
+    __syncthreads();
+    if (tid < m) {
       for (int step = 0; step < 128; ++step) {
         if (p < 0 || p >= (int32_t)n - 1) {
           mode = 0;
@@ -722,8 +800,7 @@ __global__ __launch_bounds__(kUpTile) void k_up_items(
         }
         S.far_item[side][gap] = side == 0 ? i0 : i1;
         S.far_leaf[side][gap] = side == 0 ? lo : hi;
-        const uint32_t old = __hip_atomic_fetch_add(
-            &S.cnt[gap], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const uint32_t old = lds_arrive(&S.cnt[gap]);
         if (old == 0) {
           mode = 1;
           break;
@@ -744,14 +821,15 @@ __global__ __launch_bounds__(kUpTile) void k_up_items(
           mode = 0;
           break;
         }
-        // the parent and the two words of the left-child test (up_is_left)
-        // depend only on num: three loads in flight together
-        const int32_t num = p;
-        const int32_t pl = num + 1 <= (int32_t)n - 1 ? par[n + num + 1] : -2;
-        const int32_t pn = num + 1 <= (int32_t)n - 2 ? par[num + 1] : -2;
-        self = num;
-        p = par[num];
-        side = (pl == p || pn == p) ? 0 : 1;
+        self = p;
+        if (S.node[gap] == p) {
+          p = S.node_par[gap];
+          side = S.node_side[gap];
+        } else {
+          const UpLink up = up_link(par, n, p);
+          p = up.p;
+          side = up.side;
+        }
       }
     }
     __syncthreads();
@@ -1369,37 +1447,51 @@ void launch_radix_tree(const uint32_t *keys, uint32_t n, int32_t *parents,
   hipLaunchKernelGGL(k_rt_tiles, dim3(tiles), dim3(kRtThreads), 0, s, keys, n,
                      parents, recs, cnt, last, first, tiles);
   if (n < 2) return;
+  if (tiles <= (uint32_t)kRtFewTiles) {
+    hipLaunchKernelGGL(k_rt_resolve_few, dim3(tiles), dim3(kRtFewThreads), 0, s,
+                       parents, n, recs, cnt, last, first, tiles);
+    return;
+  }
   hipLaunchKernelGGL(k_rt_scan, dim3(128), dim3(kRtScanThreads), 0, s, last,
                      first, tiles);
   hipLaunchKernelGGL(k_rt_resolve, dim3(tiles), dim3(kRtRecords), 0, s,
                      parents, n, recs, cnt, last, first, tiles);
 }
 
-uint64_t up_pass_scratch_bytes(uint32_t n) {
-  uint64_t tiles = blocks_for(n, kUpTile), items = 0, counts = 0;
-  while (true) {
-    items += tiles * kUpFront;
-    counts += tiles;
-    if (tiles == 1) break;
-    tiles = (tiles + kUpFanIn - 1) / kUpFanIn;
+// The item levels over `tiles` blocks: one block of kUpFanInMax sources costs
+// some us more than one of kUpFanIn and is taken where it saves a level (60,000
+// leaves 42.7 -> 33.6 us, 3M 154.5 -> 148.4; where it saves none, 500,000 55.4
+// -> 56.8 and 8M 296 -> 316).
+struct UpLevels {
+  uint32_t fan;
+  uint64_t tiles;  // of all levels, the leaf blocks too
+  int levels;
+};
+UpLevels up_levels_of(uint32_t tiles, uint32_t fan) {
+  UpLevels u{fan, tiles, 1};
+  for (; tiles > 1; ++u.levels) {
+    tiles = (tiles + fan - 1) / fan;
+    u.tiles += tiles;
   }
-  return 48 * items + 8 * counts;  // items, item counts, completed counts
+  return u;
+}
+UpLevels up_levels(uint32_t tiles) {
+  const UpLevels a = up_levels_of(tiles, kUpFanIn);
+  const UpLevels b = up_levels_of(tiles, kUpFanInMax);
+  return b.levels < a.levels ? b : a;
+}
+
+// Items, item counts and completed counts.
+uint64_t up_pass_scratch_bytes(uint32_t n) {
+  return (48ull * kUpFront + 8) * up_levels(blocks_for(n, kUpTile)).tiles;
 }
 
 void launch_up_pass(const int32_t *idx, const float4 *aabb,
                     const int32_t *parents, uint32_t n, float4 *nodes,
                     void *scratch, Ctl *ctl, hipStream_t s) {
   uint32_t tiles = blocks_for(n, kUpTile);
-  uint64_t total_items = 0;
-  for (uint32_t t = tiles;; t = (t + kUpFanIn - 1) / kUpFanIn) {
-    total_items += (uint64_t)t * kUpFront;
-    if (t == 1) break;
-  }
-  uint64_t total_tiles = 0;
-  for (uint32_t t = tiles;; t = (t + kUpFanIn - 1) / kUpFanIn) {
-    total_tiles += t;
-    if (t == 1) break;
-  }
+  const UpLevels u = up_levels(tiles);
+  const uint64_t total_items = u.tiles * kUpFront, total_tiles = u.tiles;
   int4 *items = static_cast<int4 *>(scratch);
   uint32_t *cnt = reinterpret_cast<uint32_t *>(items + 3 * total_items);
   uint32_t *done = cnt + total_tiles;
@@ -1408,10 +1500,10 @@ void launch_up_pass(const int32_t *idx, const float4 *aabb,
                      reinterpret_cast<const int4 *>(aabb), parents, n, nd,
                      items, cnt, done, ctl, tiles == 1 ? 1 : 0);
   while (tiles > 1) {
-    const uint32_t next = (tiles + kUpFanIn - 1) / kUpFanIn;
+    const uint32_t next = (tiles + u.fan - 1) / u.fan;
     int4 *out = items + 3 * (size_t)tiles * kUpFront;
     hipLaunchKernelGGL(k_up_items, dim3(next), dim3(kUpTile), 0, s, items,
-                       cnt, done, tiles, out, cnt + tiles, done + tiles,
+                       cnt, done, tiles, u.fan, out, cnt + tiles, done + tiles,
                        parents, n, nd, ctl, next == 1 ? 1 : 0);
     items = out;
     cnt += tiles;
