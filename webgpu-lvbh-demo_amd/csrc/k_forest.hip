@@ -300,6 +300,11 @@ __device__ __forceinline__ void forest_emit(const ForestRoot &R, uint32_t tile,
   }
 }
 
+// With segments (kSegs) every segment is a mesh of its own: positions, node ids
+// and the permutation are relative to its first leaf.  Batches of 17,555
+// triangles in 16 meshes 91 us with k_leaves / 81 here, of 713,000 in 300 152 /
+// 143, of 4.8M in 700 456 / 448; of 18M in 1,000 it turns, 1,452 / 1,462.
+//
 // Level 0: kForestLeaves sorted leaves per block.  Gathers O_TRI and the leaf
 // boxes as k_leaves does.  kStage: the nodes go out in id order through LDS,
 // four lanes per node; a mesh of at most kForestDirect leaves, whose tiles are
@@ -307,16 +312,28 @@ __device__ __forceinline__ void forest_emit(const ForestRoot &R, uint32_t tile,
 // 20.4 -> 19.7 us; one of 2^18 71.9 against 71.1 us staged, of 2^22 412
 // against 380).
 constexpr uint32_t kForestDirect = 1u << 17;
-template <bool kStage>
+template <bool kStage, bool kSegs>
 __global__ __launch_bounds__(kForestLeaves) void k_forest_leaves(
     const int4 *__restrict__ tri, const uint32_t *__restrict__ skeys,
     const int32_t *__restrict__ perm, uint32_t N, int4 *__restrict__ otri,
     int4 *__restrict__ items_out, uint32_t *__restrict__ count_out,
-    int4 *nodes, Ctl *ctl) {
+    int4 *nodes, Ctl *ctl, TreeSegs segs) {
   constexpr int T = kForestLeaves;
   __shared__ ForestLds<T> L;
   const int tid = threadIdx.x;
-  const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
+  const uint32_t gtile = xcd_tile(blockIdx.x, gridDim.x);
+  uint32_t tile = gtile;
+  if (kSegs) {  // the tile's mesh
+    const uint32_t sg = segs.tile_seg[gtile];
+    const uint32_t at = segs.seg_off[sg];
+    tile -= segs.seg_tile0[sg];
+    N = segs.seg_off[sg + 1] - at;
+    tri += 3 * (size_t)at;
+    skeys += at;
+    perm += at;
+    otri += 3 * (size_t)at;
+    nodes += 4 * (size_t)at;
+  }
   const int ts = (int)(tile * T);
   const int m = (int)min((uint32_t)T, N - (uint32_t)ts);
   const uint32_t k = (uint32_t)ts + tid;
@@ -356,7 +373,7 @@ __global__ __launch_bounds__(kForestLeaves) void k_forest_leaves(
   if (N == 1) {
     if (tid == 0) {
       write_single_leaf_node(nodes, mn, mx);
-      count_out[tile] = 0u;
+      count_out[gtile] = 0u;
     }
     return;
   }
@@ -368,26 +385,37 @@ __global__ __launch_bounds__(kForestLeaves) void k_forest_leaves(
   const ForestRoot R = forest_round<T, kStage>(
       L, m, mn, mx, d, d0, [ts](int e) { return make_int2(ts + e, ts + e); },
       (int)N, nodes, ts);
-  forest_emit(R, tile, items_out, count_out, ctl);
+  forest_emit(R, gtile, items_out, count_out, ctl);
 }
 
 // Levels >= 1: the frontiers of fan_in(prev_tiles) tiles of the level below,
 // in rounds of at most kForestItems items (the previous round's frontier
 // first, read back from the tile's own slots), as k_items.
+template <bool kSegs>
 __global__ __launch_bounds__(kForestItems) void k_forest_items(
     uint32_t N, const int4 *__restrict__ items_in,
     const uint32_t *__restrict__ count_in, uint32_t prev_tiles,
     int4 *items_out,  // written, then read back
-    uint32_t *__restrict__ count_out, int4 *nodes, Ctl *ctl) {
+    uint32_t *__restrict__ count_out, int4 *nodes, Ctl *ctl, TreeSegs segs) {
   constexpr int T = kForestItems;
   __shared__ ForestLds<T> L;
   __shared__ int2 s_range[T];
   static_assert(kFanInMax <= 64 && kFrontierMax < T, "a lane per source tile");
   const int tid = threadIdx.x, lane = tid & 63;
   const uint32_t tile = blockIdx.x;
+  uint32_t first = tile, prev0 = 0;  // its place in the mesh; source tile 0
+  if (kSegs) {
+    const uint32_t sg = segs.tile_seg[tile];
+    const uint32_t at = segs.seg_off[sg];
+    first -= segs.seg_tile0[sg];
+    prev0 = segs.prev_tile0[sg];
+    prev_tiles = segs.prev_tiles[sg];
+    N = segs.seg_off[sg + 1] - at;
+    nodes += 4 * (size_t)at;
+  }
   const uint32_t fan = fan_in(prev_tiles);
-  const uint32_t src0 = tile * fan;
-  const uint32_t nsrc = min(fan, prev_tiles - src0);
+  const uint32_t src0 = prev0 + first * fan;
+  const uint32_t nsrc = min(fan, prev_tiles - first * fan);
   // every wave scans the source counts for itself: lane s, items up to and
   // with source s
   const uint32_t own = (uint32_t)lane < nsrc
@@ -442,18 +470,24 @@ void launch_forest_level(int level, uint32_t grid, const float4 *tri,
                          uint32_t n, float4 *otri, const int4 *items_in,
                          const uint32_t *count_in, uint32_t prev_tiles,
                          int4 *items_out, uint32_t *count_out, float4 *nodes,
-                         Ctl *ctl, hipStream_t s) {
+                         Ctl *ctl, const TreeSegs &segs, hipStream_t s) {
   int4 *n4 = reinterpret_cast<int4 *>(nodes);
-  if (level > 0)
-    hipLaunchKernelGGL(k_forest_items, dim3(grid), dim3(kForestItems), 0, s, n,
-                       items_in, count_in, prev_tiles, items_out, count_out,
-                       n4, ctl);
-  else
+  const bool direct = n <= kForestDirect;
+  if (level > 0) {
     hipLaunchKernelGGL(
-        n <= kForestDirect ? k_forest_leaves<false> : k_forest_leaves<true>,
-        dim3(grid), dim3(kForestLeaves), 0, s,
-        reinterpret_cast<const int4 *>(tri), skeys, perm, n,
-        reinterpret_cast<int4 *>(otri), items_out, count_out, n4, ctl);
+        segs.tile_seg ? k_forest_items<true> : k_forest_items<false>,
+        dim3(grid), dim3(kForestItems), 0, s, n, items_in, count_in, prev_tiles,
+        items_out, count_out, n4, ctl, segs);
+  } else {
+    const auto leaves =
+        segs.tile_seg
+            ? (direct ? k_forest_leaves<false, true> : k_forest_leaves<true, true>)
+            : (direct ? k_forest_leaves<false, false> : k_forest_leaves<true, false>);
+    hipLaunchKernelGGL(leaves, dim3(grid), dim3(kForestLeaves), 0, s,
+                       reinterpret_cast<const int4 *>(tri), skeys, perm, n,
+                       reinterpret_cast<int4 *>(otri), items_out, count_out, n4,
+                       ctl, segs);
+  }
 }
 
 }  // namespace lbvh

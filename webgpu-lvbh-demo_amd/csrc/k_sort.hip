@@ -10,7 +10,8 @@
 // words per tile).
 //
 // Each pass is reduce-then-scan over tiles of kSortTile keys (kSmallSortTile
-// for a single mesh of at most kSmallSortMax keys):
+// for a single mesh of at most kSmallSortMax keys, a batch of at most
+// kBatchSmallMax):
 //   count    per-tile digit counts (pass 0's are written by the Morton
 //            kernel as it produces the keys), and their column sums;
 //   scan     one block per digit scans that digit's column of tile counts
@@ -111,19 +112,17 @@ __global__ __launch_bounds__(kSortThreads) void k_count(
   __syncthreads();
   const TileRange r = sort_tile_range(tile, n, segs, kSortThreads * kItems);
   // All of the thread's keys are loaded before any is counted, so a wave
-  // has its whole share of the tile in flight; a whole 16-byte-aligned tile
-  // with 16-byte loads (counting does not depend on which thread holds
-  // which key).
+  // has its whole share of the tile in flight; a whole tile with 16-byte
+  // loads, wherever it begins (Words4; counting does not depend on which
+  // thread holds which key).
   uint32_t k[kItems];
-  const bool vec =
-      r.end - r.begin == (uint32_t)(kSortThreads * kItems) &&
-      (reinterpret_cast<uintptr_t>(keys + r.begin) & 15u) == 0;
-  if (vec) {
-    const uint4 *k4 = reinterpret_cast<const uint4 *>(keys + r.begin);
+  if (r.end - r.begin == (uint32_t)(kSortThreads * kItems)) {
+    const Words4 *k4 = reinterpret_cast<const Words4 *>(keys + r.begin);
 #pragma unroll
     for (int q = 0; q < kItems / 4; ++q) {
-      const uint4 *src = k4 + threadIdx.x + q * kSortThreads;
-      const uint4 v = kStreamNt<kItems> ? load_nt(src) : *src;
+      const Words4 *src = k4 + threadIdx.x + q * kSortThreads;
+      const Words4 v =
+          kStreamNt<kItems> ? __builtin_nontemporal_load(src) : *src;
       k[4 * q] = v.x;
       k[4 * q + 1] = v.y;
       k[4 * q + 2] = v.z;
@@ -411,36 +410,32 @@ __global__ __launch_bounds__(kSortThreads) void k_scatter(
 
   // Warp-striped keys: wave w owns keys [wbase, wbase + 64*kItems), item
   // j of lane l sits at wbase + 64*j + l, so (j, l) order is input order.
-  // A whole 16-byte-aligned tile is loaded with 16-byte loads into the LDS
+  // A whole tile is loaded with 16-byte loads (Words4) into the LDS
   // reorder buffer (free until the reorder) and its keys read back striped:
   // 4 loads per thread instead of 16 (keys) + 16 (payloads).  Payloads stay
   // in s_vals (at the striped position) until the ranking is done, so they
   // hold no registers while it runs.
   const uint32_t wbase = r.begin + wave * 64 * kItems;
   uint32_t key[kItems];
-  const bool vec =
-      r.end - r.begin == (uint32_t)kTile &&
-      ((reinterpret_cast<uintptr_t>(keys_in + r.begin) |
-        (kFirst ? 0u : reinterpret_cast<uintptr_t>(vals_in + r.begin))) &
-       15u) == 0;
-  if (vec) {
-    const uint4 *k4 = reinterpret_cast<const uint4 *>(keys_in + r.begin);
-    const int4 *v4 = reinterpret_cast<const int4 *>(vals_in + r.begin);
-    uint4 kq[kItems / 4];
-    int4 vq[kItems / 4];
+  if (r.end - r.begin == (uint32_t)kTile) {
+    const Words4 *k4 = reinterpret_cast<const Words4 *>(keys_in + r.begin);
+    const Words4 *v4 = reinterpret_cast<const Words4 *>(vals_in + r.begin);
+    Words4 kq[kItems / 4], vq[kItems / 4];
 #pragma unroll
     for (int q = 0; q < kItems / 4; ++q) {
-      kq[q] = kStreamNt<kItems> ? load_nt(k4 + tid + q * kSortThreads)
-                                : k4[tid + q * kSortThreads];
+      const int e = tid + q * kSortThreads;
+      kq[q] = kStreamNt<kItems> ? __builtin_nontemporal_load(k4 + e) : k4[e];
       if (!kFirst)
-        vq[q] = kStreamNt<kItems> ? load_nt(v4 + tid + q * kSortThreads)
-                                  : v4[tid + q * kSortThreads];
+        vq[q] = kStreamNt<kItems> ? __builtin_nontemporal_load(v4 + e) : v4[e];
     }
 #pragma unroll
     for (int q = 0; q < kItems / 4; ++q) {
-      reinterpret_cast<uint4 *>(s_keys)[tid + q * kSortThreads] = kq[q];
+      const int e = tid + q * kSortThreads;
+      reinterpret_cast<uint4 *>(s_keys)[e] =
+          make_uint4(kq[q].x, kq[q].y, kq[q].z, kq[q].w);
       if (!kFirst)
-        reinterpret_cast<int4 *>(s_vals)[tid + q * kSortThreads] = vq[q];
+        reinterpret_cast<int4 *>(s_vals)[e] =
+            make_int4((int)vq[q].x, (int)vq[q].y, (int)vq[q].z, (int)vq[q].w);
     }
     __syncthreads();
 #pragma unroll
@@ -657,8 +652,8 @@ void launch_sort_pass(int bits, int pass, const uint32_t *keys_in,
   if (tiles == 0) return;
   const SortSegs one{};
   const SortSegs &sg = segs ? *segs : one;
-  // a batched sort keeps kSortTile tiles; a single mesh's tile follows n
-  const bool small = !segs && sort_items(n) == kSmallSortItems;
+  // a single mesh's tile follows n
+  const bool small = (segs ? segs->items : sort_items(n)) == kSmallSortItems;
 #define LBVH_SORT_PASS(B, I)                                                 \
   sort_pass<B, I>(pass, keys_in, vals_in, keys_out, vals_out, n, tiles, cnt, \
                   off, counted, ctl, s, sg, segs != nullptr, num_segs,       \

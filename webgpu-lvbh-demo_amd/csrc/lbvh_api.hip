@@ -67,7 +67,8 @@ struct lbvh_ctx {
       b_bounds, b_tree_items, b_tree_counts, b_table, b_cen;
   struct BatchPlan {
     std::vector<uint32_t> offsets;
-    int tile = 0, bits = kRadixBits;
+    int tile = 0, bits = kRadixBits, items = kSortItems;
+    bool forest = false;
     uint32_t S = 0, total = 0, sort_tiles = 0;
     int levels = 0;
     std::vector<uint32_t> level_tiles;
@@ -475,6 +476,12 @@ TreePlan tree_plan(const lbvh_ctx *ctx, uint32_t n) {
   return {tile, false};
 }
 
+// Keys per thread of a batched sort of n keys in all: the small tile as for a
+// single mesh, but not under an HBM budget (four times the tiles' counts).
+int batch_sort_items(const lbvh_ctx *ctx, uint32_t n) {
+  return ctx->budget == 0 && n <= kBatchSmallMax ? kSmallSortItems : kSortItems;
+}
+
 int bits_for(const lbvh_ctx *ctx, uint32_t n) {
   return tuned_for(ctx->sort_bits, ctx->sort_bits_fixed, ctx->tune_bits, n,
                    untuned_bits(n));
@@ -581,7 +588,7 @@ void run_tree(lbvh_ctx *ctx, int4 *items, uint32_t *counts, const float *tri,
     if (plan.forest)
       launch_forest_level(L, grid[L], t4, skeys, perm, n, o4, items_in,
                           counts + prev, below, items_out, counts + base,
-                          nodes, ctx->ctl, ctx->stream);
+                          nodes, ctx->ctl, TreeSegs{}, ctx->stream);
     else
       launch_tree_level(L, plan.tile, grid[L], t4, skeys, perm, n, o4, items_in,
                         counts + prev, below, items_out, counts + base, nodes,
@@ -749,7 +756,11 @@ int make_plan(lbvh_ctx *ctx, const uint32_t *offsets, uint32_t S) {
   auto &P = ctx->plan;
   uint32_t big = 0;
   for (uint32_t k = 0; k < S; ++k) big = std::max(big, offsets[k + 1] - offsets[k]);
-  if (P.S == S && P.tile == tile_for(ctx, big) &&
+  // the trees' levels run together: k_forest.hip's up to as many leaves in all
+  TreePlan plan = tree_plan(ctx, offsets[S]);
+  if (!plan.forest) plan.tile = tile_for(ctx, big);
+  const int items = batch_sort_items(ctx, offsets[S]);
+  if (P.S == S && P.items == items && P.tile == plan.tile && P.forest == plan.forest &&
       P.bits == bits_for(ctx, offsets[S]) &&
       std::equal(P.offsets.begin(), P.offsets.end(), offsets) &&
       P.offsets.size() == (size_t)S + 1)
@@ -757,10 +768,9 @@ int make_plan(lbvh_ctx *ctx, const uint32_t *offsets, uint32_t S) {
   drop_plan(ctx);
   P.offsets.assign(offsets, offsets + S + 1);
   P.S = S;
-  uint32_t largest = 0;
-  for (uint32_t k = 0; k < S; ++k)
-    largest = std::max(largest, offsets[k + 1] - offsets[k]);
-  P.tile = tile_for(ctx, largest);
+  P.tile = plan.tile;
+  P.forest = plan.forest;
+  P.items = items;
   // one segmented sort runs over all the keys: its digit width is that of
   // a sort of the total
   P.bits = bits_for(ctx, offsets[S]);
@@ -778,7 +788,7 @@ int make_plan(lbvh_ctx *ctx, const uint32_t *offsets, uint32_t S) {
   for (uint32_t k = 0; k < S; ++k) {
     const uint32_t n = offsets[k + 1] - offsets[k];
     seg_tile0[k] = (uint32_t)tile_seg.size();
-    for (uint32_t j = 0; j < batch_sort_tiles(n); ++j) tile_seg.push_back(k);
+    for (uint32_t j = 0; j < batch_sort_tiles(n, P.items); ++j) tile_seg.push_back(k);
     if (n) {
       grid_k[k].resize(kMaxTreeLevels);
       levels_k[k] = tree_levels(n, P.tile, grid_k[k].data());
@@ -824,7 +834,8 @@ void enqueue_batch(lbvh_ctx *ctx, const float *tri, bool have_bounds,
   const uint32_t *T = static_cast<const uint32_t *>(ctx->b_table.ptr);
   uint32_t *ord = static_cast<uint32_t *>(ctx->b_ord.ptr);
   const float4 *t4 = reinterpret_cast<const float4 *>(tri);
-  const SortSegs ss{T + P.o_tile_seg, T + P.o_seg_tile0, T + P.o_seg_off};
+  const SortSegs ss{T + P.o_tile_seg, T + P.o_seg_tile0, T + P.o_seg_off,
+                    P.items};
   launch_batch_prologue(ord, P.S, !have_bounds, ctx->ctl, ctx->stream);
   float *cen = have_bounds ? nullptr : static_cast<float *>(ctx->b_cen.ptr);
   if (!have_bounds)
@@ -856,12 +867,20 @@ void enqueue_batch(lbvh_ctx *ctx, const float *tri, bool have_bounds,
     if (P.level_tiles[L] == 0) break;
     const TreeSegs ts{T + P.o_ltile_seg[L], T + P.o_lseg_tile0[L],
                       T + P.o_seg_off, T + P.o_lprev0[L], T + P.o_lprev_n[L]};
-    launch_tree_level(L, P.tile, P.level_tiles[L], t4, out, vout, P.total,
-                      reinterpret_cast<float4 *>(tri_out),
-                      items + kItemInt4 * kTreeFrontier * prev, counts + prev, 0u,
-                      items + kItemInt4 * kTreeFrontier * base, counts + base,
-                      static_cast<float4 *>(bvh_out), ctx->ctl, ts,
-                      ctx->stream);
+    const int4 *items_in = items + kItemInt4 * kTreeFrontier * prev;
+    int4 *items_out = items + kItemInt4 * kTreeFrontier * base;
+    if (P.forest)
+      launch_forest_level(L, P.level_tiles[L], t4, out, vout, P.total,
+                          reinterpret_cast<float4 *>(tri_out), items_in,
+                          counts + prev, 0u, items_out, counts + base,
+                          static_cast<float4 *>(bvh_out), ctx->ctl, ts,
+                          ctx->stream);
+    else
+      launch_tree_level(L, P.tile, P.level_tiles[L], t4, out, vout, P.total,
+                        reinterpret_cast<float4 *>(tri_out), items_in,
+                        counts + prev, 0u, items_out, counts + base,
+                        static_cast<float4 *>(bvh_out), ctx->ctl, ts,
+                        ctx->stream);
     prev = base;
     base += P.level_tiles[L];
   }

@@ -42,6 +42,10 @@ constexpr int kSortTile = kSortThreads * kSortItems;  // 4096 keys per tile
 constexpr int kSmallSortItems = 4;
 constexpr int kSmallSortTile = kSortThreads * kSmallSortItems;  // 1024 keys
 constexpr uint32_t kSmallSortMax = 1u << 20;
+// Batched sorts of at most this many keys in all use the small tile too: 17,555
+// keys in 16 meshes 81.6 / 61.9 us a batch, 713,000 in 300 141 / 107, 4.8M in
+// 700 450 / 429 (4,096 / 1,024 keys); 18M in 1,000 turns, 1,438 / 1,535.
+constexpr uint32_t kBatchSmallMax = 1u << 23;
 
 constexpr int kTreeTileDefault = 1024;  // leaves per tile of the fused up pass
 constexpr int kMaxTreeLevels = 16;      // agglomeration levels (6 at 2^24, T=1024)
@@ -119,13 +123,14 @@ void launch_copy_bounds(const Ctl *ctl, float *out, hipStream_t s);
 
 // k_sort.hip
 // Segments of a batched sort (all null: one segment [0, n)).  Tiles of
-// kSortTile keys never straddle segments; tile_seg maps each tile to its
+// kSortThreads x items keys never straddle segments; tile_seg maps each tile to its
 // segment, seg_tile0 gives a segment's first tile, seg_off its first key
 // (S+1 entries).
 struct SortSegs {
   const uint32_t *tile_seg;
   const uint32_t *seg_tile0;
   const uint32_t *seg_off;
+  int items;  // keys per thread of the tiles
 };
 // One digit pass of `bits`-bit digits (kRadixBits or kWideBits) over
 // `tiles` sort tiles (pass 0 takes the position in the segment as payload
@@ -142,8 +147,7 @@ void launch_sort_pass(int bits, int pass, const uint32_t *keys_in,
                       uint32_t *cnt, uint32_t *off, bool counted, Ctl *ctl,
                       hipStream_t s, const SortSegs *segs = nullptr,
                       uint32_t num_segs = 0, int key_bits = kKeyBits);
-// Keys per thread and tiles of a single-mesh sort of n keys (batched sorts
-// always use kSortTile: batch_sort_tiles).
+// Keys per thread and tiles of a single-mesh sort of n keys.
 inline int sort_items(uint32_t n) {
   return n <= kSmallSortMax ? kSmallSortItems : kSortItems;
 }
@@ -151,8 +155,10 @@ inline uint32_t sort_tiles(uint32_t n) {
   const uint32_t t = (uint32_t)(kSortThreads * sort_items(n));
   return (n + t - 1) / t;
 }
-inline uint32_t batch_sort_tiles(uint32_t n) {
-  return (n + kSortTile - 1) / kSortTile;
+// Tiles of one mesh of a batched sort.
+inline uint32_t batch_sort_tiles(uint32_t n, int items) {
+  const uint32_t t = (uint32_t)(kSortThreads * items);
+  return (n + t - 1) / t;
 }
 // The sort of a single key: perm[0] = 0 and sorted[0] = keys[0] (sorted may
 // be keys).  A one-thread kernel, so that a build stays kernels only.
@@ -239,7 +245,7 @@ void launch_tree_level(int level, int tile, uint32_t grid, const float4 *tri,
                        Ctl *ctl, const TreeSegs &segs, hipStream_t s);
 
 // k_forest.hip
-// One agglomeration level of a mesh of at most kForestMax leaves, over leaf
+// One agglomeration level of at most kForestMax leaves in all, over leaf
 // tiles of kForestTile: the arguments, items and level plan of
 // launch_tree_level.  Refits, this against the best leaf tile of k_leaves:
 // 1,500 leaves 9.4 / 17.3 us, 2^16 16.3 / 24.5, 2^18 24.7 / 37, 2^20 63 / 72
@@ -252,7 +258,7 @@ void launch_forest_level(int level, uint32_t grid, const float4 *tri,
                          uint32_t n, float4 *otri, const int4 *items_in,
                          const uint32_t *count_in, uint32_t prev_tiles,
                          int4 *items_out, uint32_t *count_out, float4 *nodes,
-                         Ctl *ctl, hipStream_t s);
+                         Ctl *ctl, const TreeSegs &segs, hipStream_t s);
 
 // k_batch.hip
 void launch_batch_prologue(uint32_t *seg_ord, uint32_t num_segs,
