@@ -41,3 +41,11 @@ def test_build(ctx, lb, ora, n, bounds):
         assert np.array_equal(bvh, wb)
         assert np.array_equal(otri.view(np.uint32), wo.view(np.uint32))
         assert np.array_equal(ctx.build_arrays(tri, b)[0], wb)  # keys in scratch
+
+
+# where the tile grows: one tile of 512, 1,024 or 2,048 keys, then several
+@pytest.mark.parametrize("n", [511, 512, 513, 1023, 1024, 1025, 1537, 3000, 4096, 4097, 8193, 16383])
+def test_small_tiles(ctx, lb, ora, n):
+    test_sort(ctx, n)
+    for bounds in ("gpu", "caller"):
+        test_build(ctx, lb, ora, n, bounds)

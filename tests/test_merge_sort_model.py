@@ -69,7 +69,7 @@ def chunk_positions(keys, n, c0, run_log, group_log):
     run = c0 >> run_log
     runs = 1 << group_log
     g0 = run & ~(runs - 1)
-    x, have = run_log - TILE_LOG, n >> SAMPLE_LOG
+    x, have = max(run_log - TILE_LOG, 0), n >> SAMPLE_LOG  # a short run has fewer samples
     assert x <= 6
     rank, widest, rng = np.zeros(64, np.int64), 0, np.random.default_rng(c0)
     for s in range(g0, g0 + runs):
@@ -159,7 +159,7 @@ def test_merge_sort_is_the_stable_sort(n, full):
         assert np.array_equal(k, keys[want])
 
 
-@pytest.mark.parametrize("run_log", [7, 10, 13])
+@pytest.mark.parametrize("run_log", [6, 7, 10, 13])
 def test_uneven_runs_take_every_search(run_log):
     """One and two readings of the samples, narrow and wide windows."""
     rng = np.random.default_rng(7)

@@ -7,7 +7,8 @@
 // A small sort is a chain of short kernels, each of a few microseconds of
 // latency whatever its size: keys and radix passes of 64K triangles took nine
 // launches and 43 us.  Here they are two and 18 us:
-//   k_tile_sort    a block sorts kMsTile keys in LDS (10-11 us).  In a build
+//   k_tile_sort    a block sorts up to kMsTile keys in LDS (10-11 us; small
+//                  sorts take smaller tiles, tile_log).  In a build
 //                  it makes the keys itself, from the box centres or the
 //                  triangles, so the Morton pass is this kernel too.
 //   k_merge        merges groups of 8, 16 or 32 sorted runs: every key finds
@@ -22,9 +23,7 @@
 
 namespace lbvh {
 
-constexpr int kMsThreads = 1024;
-constexpr int kMsPer = kMsTile / kMsThreads;
-static_assert(kMsPer == 2, "a thread's pair starts the runs of two");
+constexpr int kMsPer = 2;  // keys per thread: a pair starts the runs of two
 constexpr int kMsWave = 64 * kMsPer;  // keys per wave
 
 // Every kSample-th sorted key also goes to a compact array, which the merge
@@ -44,9 +43,9 @@ __device__ __forceinline__ uint32_t lane_value(uint32_t v, int lane) {
 // the sibling run (keys equal to it count when the sibling comes first, so
 // equal keys keep their order).  Runs inside a wave need no block barrier: a
 // wave's LDS operations complete in issue order.
-template <int kLen, bool kFull>
-__device__ __forceinline__ void merge_round(uint32_t (*s_key)[kMsTile],
-                                            uint16_t (*s_idx)[kMsTile],
+template <int kLen, bool kFull, int kTile>
+__device__ __forceinline__ void merge_round(uint32_t (*s_key)[kTile],
+                                            uint16_t (*s_idx)[kTile],
                                             int &cur) {
   const uint32_t p0 = 2 * threadIdx.x;
   const uint32_t sib = (p0 ^ kLen) & ~(uint32_t)(kLen - 1);
@@ -91,18 +90,19 @@ __device__ __forceinline__ void ms_box_centre(const float4 *__restrict__ t,
   for (int k = 0; k < 3; ++k) ce[k] = __fmul_rn(__fadd_rn(mx[k], mn[k]), 0.5f);
 }
 
-template <int kSrc, bool kFull>
-__global__ __launch_bounds__(kMsThreads) void k_tile_sort(
+template <int kSrc, bool kFull, int kTile>
+__global__ __launch_bounds__(kTile / kMsPer) void k_tile_sort(
     MergeKeys src, uint32_t n, uint32_t *keys_out,
     int32_t *__restrict__ idx_out, uint32_t *__restrict__ smp_out) {
-  __shared__ __align__(16) uint32_t s_key[2][kMsTile];
-  __shared__ __align__(16) uint16_t s_idx[2][kMsTile];
+  constexpr int kThreads = kTile / kMsPer;
+  __shared__ __align__(16) uint32_t s_key[2][kTile];
+  __shared__ __align__(16) uint16_t s_idx[2][kTile];
   __shared__ float s_b[8];
   // past every key in order: real keys with this value come before
   constexpr uint32_t kPast = kFull ? 0xFFFFFFFFu : 0x7FFFFFFFu;
   const uint32_t tid = threadIdx.x;
-  const uint32_t base = xcd_tile(blockIdx.x, gridDim.x) * (uint32_t)kMsTile;
-  const uint32_t valid = min(n - base, (uint32_t)kMsTile);
+  const uint32_t base = xcd_tile(blockIdx.x, gridDim.x) * (uint32_t)kTile;
+  const uint32_t valid = min(n - base, (uint32_t)kTile);
   const uint32_t p0 = 2 * tid, i0 = base + p0;
   uint32_t key[2] = {kPast, kPast};
   if (kSrc == kSrcKeys) {
@@ -152,9 +152,8 @@ __global__ __launch_bounds__(kMsThreads) void k_tile_sort(
         if (tid == 0)
           for (int k = 0; k < 6; ++k) s_b[k] = v[k];
       } else {
-        // wave c folds component c of the partials, kFoldPer loads in flight
-        const uint32_t c = tid >> 6;
-        if (c < 6) {
+        // a wave folds a component of the partials, kFoldPer loads in flight
+        for (uint32_t c = tid >> 6; c < 6; c += kThreads / 64) {
           constexpr uint32_t kFoldPer = kBoundsBlocks / 64;
           const float *part = reinterpret_cast<const float *>(src.partials) +
                               (c < 3 ? c : c + 1);
@@ -195,7 +194,7 @@ __global__ __launch_bounds__(kMsThreads) void k_tile_sort(
       swap ? (p0 << 16) | (p0 + 1) : ((p0 + 1) << 16) | p0;
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
-#define LBVH_ROUND(L) merge_round<L, kFull>(s_key, s_idx, cur)
+#define LBVH_ROUND(L) merge_round<L, kFull, kTile>(s_key, s_idx, cur)
   LBVH_ROUND(2);
   LBVH_ROUND(4);
   LBVH_ROUND(8);
@@ -205,13 +204,14 @@ __global__ __launch_bounds__(kMsThreads) void k_tile_sort(
   __syncthreads();
   if (valid > 128) LBVH_ROUND(128);
   if (valid > 256) LBVH_ROUND(256);
-  if (valid > 512) LBVH_ROUND(512);
-  if (valid > 1024) LBVH_ROUND(1024);
+  if (kTile > 512 && valid > 512) LBVH_ROUND(512 % kTile);
+  if (kTile > 1024 && valid > 1024) LBVH_ROUND(1024 % kTile);
 #undef LBVH_ROUND
-  static_assert(kMsTile == 2048 && kMsWave == 128, "the rounds above");
+  static_assert(kTile >= 512 && kTile <= 2048 && kMsWave == 128,
+                "the rounds above");
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
-    const uint32_t p = e * kMsThreads + tid;
+    const uint32_t p = e * kThreads + tid;
     if (p < valid) {
       const uint32_t k = s_key[cur][p];
       keys_out[base + p] = k;
@@ -282,7 +282,8 @@ __global__ __launch_bounds__(kMergeThreads) void k_merge(
     const uint32_t at = min(i, n - 1);  // past the end: the last key again
     key = keys_in[at];
     if (sub == 0) val = idx_in[at];
-    const int x = run_log - kMsTileLog;  // every 2^x-th sample: 64 per run
+    // every 2^x-th sample: 64 per run (fewer of a run below 2^kMsTileLog)
+    const int x = max(run_log - kMsTileLog, 0);
     const uint32_t have = n >> kSampleLog;
     uint32_t smp[kPer], len[kPer];
 #pragma unroll
@@ -441,6 +442,19 @@ __global__ __launch_bounds__(kMergeThreads) void k_merge(
   }
 }
 
+// Keys per tile, 2^this.  A block's rounds take 10-11 us at 2,048 keys, 16
+// waves on one CU, and less with fewer on more CUs, while the merge of all the
+// tiles stays one round of a few runs.  Builds in us by tile of 2,048 / 1,024 /
+// 512 keys: 2,500 triangles 26.3 / 23.4 / 22.0, 5,000 26.9 / 23.3 / 23.1
+// (heightfield 27.1 / 24.3 / 24.7), 16,384 31.1 / 28.7 / 28.8 (31.9 / 30.5 /
+// 32.1); heightfields of 20,000 turn, 34.0 / 34.5 / 34.8.  One tile needs no
+// merge: 1,024 triangles with caller bounds 16.2 / 15.4 / 17.7.
+static int tile_log(const MergeKeys &src, uint32_t n) {
+  if (n <= 1u << 10) return n <= 1u << 9 ? 9 : 10;
+  if (src.whole) return kMsTileLog;
+  return n <= 8u << 9 ? 9 : n <= 16u << 10 ? 10 : kMsTileLog;
+}
+
 // The merge rounds of a sort of n keys: up to 32 tiles merge in one round,
 // four waves per 64 keys (their searches are the round's latency); more merge
 // 8 runs at a time, a wave per 64 keys, before a last round of up to 16.
@@ -449,9 +463,9 @@ struct MergeRound {
   int group_log;        // 2^group_log of them merged together
 };
 constexpr int kMaxMergeRounds = 8;
-static int merge_plan(uint32_t n, MergeRound *r) {
-  uint32_t runs = (n + kMsTile - 1) / kMsTile;
-  int rounds = 0, log = kMsTileLog;
+static int merge_plan(const MergeKeys &src, uint32_t n, MergeRound *r) {
+  int rounds = 0, log = tile_log(src, n);
+  uint32_t runs = (n + (1u << log) - 1) >> log;
   while (runs > 1) {
     int g = 3;
     if (runs <= (rounds ? 16u : 32u))
@@ -474,26 +488,33 @@ void launch_tile_sort(const MergeKeys &src, uint32_t n, uint32_t *keys_tmp,
                       uint32_t *samples, hipStream_t s) {
   // the tile sort and every round alternate buffers, the last one writes out
   MergeRound rounds[kMaxMergeRounds];
-  const bool odd = merge_plan(n, rounds) % 2;
+  const bool odd = merge_plan(src, n, rounds) % 2;
   uint32_t *k = odd ? keys_tmp : keys_out;
   int32_t *v = odd ? idx_tmp : idx_out;
-#define LBVH_TILE_SORT(SRC, FULL)                                         \
-  hipLaunchKernelGGL((k_tile_sort<SRC, FULL>),                            \
-                     dim3((n + kMsTile - 1) / kMsTile), dim3(kMsThreads), \
-                     0, s, src, n, k, v, samples)
-  if (src.keys) LBVH_TILE_SORT(kSrcKeys, true);
-  else if (src.cen) LBVH_TILE_SORT(kSrcCentres, false);
-  else if (src.whole) LBVH_TILE_SORT(kSrcWholeMesh, false);
-  else LBVH_TILE_SORT(kSrcTriangles, false);
+  const int log = tile_log(src, n);
+#define LBVH_TILE_SORT(SRC, FULL, T)                                      \
+  hipLaunchKernelGGL((k_tile_sort<SRC, FULL, T>), dim3((n + T - 1) / T),  \
+                     dim3(T / kMsPer), 0, s, src, n, k, v, samples)
+#define LBVH_TILE_SORTS(SRC, FULL)                       \
+  do {                                                   \
+    if (log == 9) LBVH_TILE_SORT(SRC, FULL, 512);        \
+    else if (log == 10) LBVH_TILE_SORT(SRC, FULL, 1024); \
+    else LBVH_TILE_SORT(SRC, FULL, kMsTile);             \
+  } while (0)
+  if (src.keys) LBVH_TILE_SORTS(kSrcKeys, true);
+  else if (src.cen) LBVH_TILE_SORTS(kSrcCentres, false);
+  else if (src.whole) LBVH_TILE_SORTS(kSrcWholeMesh, false);
+  else LBVH_TILE_SORTS(kSrcTriangles, false);
+#undef LBVH_TILE_SORTS
 #undef LBVH_TILE_SORT
 }
 
 template <bool kFull>
-static void merge_rounds(uint32_t n, uint32_t *keys_tmp, int32_t *idx_tmp,
-                         uint32_t *keys_out, int32_t *idx_out,
+static void merge_rounds(const MergeKeys &src, uint32_t n, uint32_t *keys_tmp,
+                         int32_t *idx_tmp, uint32_t *keys_out, int32_t *idx_out,
                          uint32_t *samples, hipStream_t s) {
   MergeRound rounds[kMaxMergeRounds];
-  const int count = merge_plan(n, rounds);
+  const int count = merge_plan(src, n, rounds);
   const bool odd = count % 2;
   uint32_t *smp = samples, *smp2 = samples + merge_samples(n);
   uint32_t *k = odd ? keys_tmp : keys_out, *k2 = odd ? keys_out : keys_tmp;
@@ -521,9 +542,9 @@ void launch_merge_rounds(const MergeKeys &src, uint32_t n, uint32_t *keys_tmp,
                          int32_t *idx_tmp, uint32_t *keys_out,
                          int32_t *idx_out, uint32_t *samples, hipStream_t s) {
   if (src.keys)
-    merge_rounds<true>(n, keys_tmp, idx_tmp, keys_out, idx_out, samples, s);
+    merge_rounds<true>(src, n, keys_tmp, idx_tmp, keys_out, idx_out, samples, s);
   else
-    merge_rounds<false>(n, keys_tmp, idx_tmp, keys_out, idx_out, samples, s);
+    merge_rounds<false>(src, n, keys_tmp, idx_tmp, keys_out, idx_out, samples, s);
 }
 
 }  // namespace lbvh
