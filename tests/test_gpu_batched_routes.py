@@ -10,15 +10,19 @@ pytestmark = pytest.mark.gpu
 
 SMALL = [1, 1023, 1024, 1025, 3, 4096, 4097, 4095, 255, 257, 16385, 2, 70001]
 LARGE = SMALL + [262144, 131073, 100003] * 16  # 7.9M
+# meshes of more sort tiles than bounds blocks, and empty ones
+FEW = [3, 600001, 0, 0, 1030, 524289, 0, 7] + [0] * 300 + [2]
 LARGER = LARGE + [262144, 262143]              # past 2^23
 
 
 @pytest.mark.parametrize("bits", [8, 10])
 @pytest.mark.parametrize("with_bounds", [False, True])
-@pytest.mark.parametrize("sizes", [SMALL, LARGE, LARGER], ids=["small", "large", "larger"])
+@pytest.mark.parametrize("sizes", [SMALL, FEW, LARGE, LARGER], ids=["small", "few", "large", "larger"])
 def test_routes_agree(lb, ora, sizes, with_bounds, bits):
     meshes, offsets, tri = make_batch(lb, sizes, 300)
-    bounds = np.concatenate([lb.wl_bounds(m) for m in meshes]) if with_bounds else None
+    bounds = None
+    if with_bounds:
+        bounds = np.concatenate([lb.wl_bounds(m) if len(m) else np.zeros(6, np.float32) for m in meshes])
     outs = []
     for budget in (0, 64 << 30):
         with lb.Context(0, hbm_budget=budget) as c:
@@ -29,6 +33,8 @@ def test_routes_agree(lb, ora, sizes, with_bounds, bits):
     bvh, otri, sk, pm = outs[0]
     for k in list(range(len(SMALL))) + [len(sizes) - 1]:
         a, b = int(offsets[k]), int(offsets[k + 1])
+        if a == b:
+            continue
         wb, wo, wsk, wpm = ora.build(meshes[k], None if bounds is None else bounds[6 * k:6 * k + 6], 0)
         assert np.array_equal(sk[a:b], wsk) and np.array_equal(pm[a:b], wpm), k
         assert np.array_equal(bvh[64 * a:64 * b], wb), k

@@ -242,22 +242,31 @@ __global__ __launch_bounds__(kThreads) void k_scan_columns(
 // its tile t starts at seg_off + (the segment's keys with a smaller digit)
 // + (digit-d keys in the segment's earlier tiles).  The counts are
 // tile-major, so the segment's are one contiguous run of tiles * R words:
-// thread t owns digits [t * kDpt, (t + 1) * kDpt) and reads them tile after
-// tile (each tile's R words in one coalesced sweep of the block), kUnroll
-// tiles in flight; it sums them over the segment, the block scans the sums
-// into bases, and the thread writes its running positions.  An empty
-// segment has no tiles.
-template <int kBits>
-__global__ __launch_bounds__(kSortThreads) void k_seg_scan(
+// the block's kSegGroups groups of kSortThreads threads take a part of the
+// tiles each, thread t of a group its digits [t * kDpt, (t + 1) * kDpt), tile
+// after tile (each tile's R words in one coalesced sweep of the group), kUnroll
+// tiles in flight; the groups' sums and a scan over the digits give each its
+// first positions.  An empty segment has no tiles.  One group takes 9 us for a
+// mesh of 64 tiles, the chain of its loads, four 5; but four where blocks fill
+// the chip cost more (300 meshes 4.8 against 3.6 us, 1,000 8.8 against 6.2).
+constexpr uint32_t kFewSegs = 256;  // at most so many segments: four groups
+template <int kBits, int kSegGroups>
+__global__ __launch_bounds__(kSegGroups *kSortThreads) void k_seg_scan(
     const uint32_t *__restrict__ cnt, uint32_t *__restrict__ off,
     uint32_t tiles, SortSegs segs, uint32_t num_segs) {
   using D = Digits<kBits>;
   constexpr int kUnroll = 8;
   __shared__ uint32_t s_wsum[16];
+  __shared__ uint32_t s_sum[kSegGroups][kSegGroups > 1 ? D::kR : 1];
+  __shared__ uint32_t s_base[kSegGroups > 1 ? D::kR : 1];
   const uint32_t sg = blockIdx.x;
-  const uint32_t t0 = segs.seg_tile0[sg];
-  const uint32_t t1 = (sg + 1 < num_segs) ? segs.seg_tile0[sg + 1] : tiles;
-  const uint32_t d0 = threadIdx.x * D::kDpt;
+  const uint32_t first = segs.seg_tile0[sg];
+  const uint32_t all = ((sg + 1 < num_segs) ? segs.seg_tile0[sg + 1] : tiles) - first;
+  const uint32_t group = threadIdx.x / kSortThreads;
+  const uint32_t per = (all + kSegGroups - 1) / kSegGroups;
+  const uint32_t t0 = first + min(group * per, all);
+  const uint32_t t1 = first + min(group * per + per, all);
+  const uint32_t d0 = (threadIdx.x % kSortThreads) * D::kDpt;
   uint32_t total[D::kDpt];
 #pragma unroll
   for (int i = 0; i < D::kDpt; ++i) total[i] = 0u;
@@ -274,10 +283,37 @@ __global__ __launch_bounds__(kSortThreads) void k_seg_scan(
       for (int i = 0; i < D::kDpt; ++i) total[i] += c[u][i];
   }
   uint32_t run[D::kDpt];
-  digit_prefix<kBits>(total, run, s_wsum);
-  const uint32_t first = segs.seg_off[sg];
+  if (kSegGroups == 1) {
+    digit_prefix<kBits>(total, run, s_wsum);
+  } else {
 #pragma unroll
-  for (int i = 0; i < D::kDpt; ++i) run[i] += first;
+    for (int i = 0; i < D::kDpt; ++i) s_sum[group][d0 + i] = total[i];
+    __syncthreads();
+    // the segment's totals in the first group (the others scan nothing), and
+    // this group's digits in the groups before it
+    uint32_t before[D::kDpt], base[D::kDpt];
+#pragma unroll
+    for (int i = 0; i < D::kDpt; ++i) {
+      uint32_t sum = 0;
+      before[i] = 0;
+#pragma unroll
+      for (int g = 0; g < kSegGroups; ++g) {
+        if ((uint32_t)g == group) before[i] = sum;
+        sum += s_sum[g][d0 + i];
+      }
+      total[i] = group == 0 ? sum : 0u;
+    }
+    digit_prefix<kBits>(total, base, s_wsum);
+    if (group == 0) {
+#pragma unroll
+      for (int i = 0; i < D::kDpt; ++i) s_base[d0 + i] = base[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < D::kDpt; ++i) run[i] = s_base[d0 + i] + before[i];
+  }
+#pragma unroll
+  for (int i = 0; i < D::kDpt; ++i) run[i] += segs.seg_off[sg];
   for (uint32_t t = t0; t < t1; t += kUnroll) {
     uint32_t c[kUnroll][D::kDpt];
 #pragma unroll
@@ -607,8 +643,14 @@ void sort_pass(int pass, const uint32_t *keys_in, const int32_t *vals_in,
   const int small = !segmented && tiles <= kSmallScanTiles;
   const uint32_t *offs = small ? cnt : off;
   if (segmented) {
-    hipLaunchKernelGGL(k_seg_scan<kBits>, dim3(num_segs), dim3(kSortThreads),
-                       0, s, cnt, off, tiles, sg, num_segs);
+    if (num_segs <= kFewSegs && tiles > 4 * num_segs)
+      hipLaunchKernelGGL((k_seg_scan<kBits, 4>), dim3(num_segs),
+                         dim3(4 * kSortThreads), 0, s, cnt, off, tiles, sg,
+                         num_segs);
+    else
+      hipLaunchKernelGGL((k_seg_scan<kBits, 1>), dim3(num_segs),
+                         dim3(kSortThreads), 0, s, cnt, off, tiles, sg,
+                         num_segs);
   } else if (!small) {
     bases_from = hist;
     if (tiles <= kScanSmall / 4)

@@ -63,8 +63,8 @@ struct lbvh_ctx {
   DevBuf cen;                           // triangle box centres (GPU bounds)
   // batched builds: scratch, and the plan (tile tables + captured graph) of
   // the last batch layout
-  DevBuf b_keys_a, b_keys_b, b_idx_a, b_idx_b, b_digits, b_ord,
-      b_bounds, b_tree_items, b_tree_counts, b_table, b_cen;
+  DevBuf b_keys_a, b_keys_b, b_idx_a, b_idx_b, b_digits, b_bounds,
+      b_tree_items, b_tree_counts, b_table, b_cen;
   struct BatchPlan {
     std::vector<uint32_t> offsets;
     int tile = 0, bits = kRadixBits, items = kSortItems;
@@ -74,6 +74,8 @@ struct lbvh_ctx {
     std::vector<uint32_t> level_tiles;
     // u32 offsets of the tables inside b_table
     uint64_t o_seg_off = 0, o_tile_seg = 0, o_seg_tile0 = 0;
+    uint64_t o_blk_seg = 0, o_seg_blk0 = 0;
+    uint32_t bounds_blocks = 0;
     std::vector<uint64_t> o_ltile_seg, o_lseg_tile0, o_lprev0, o_lprev_n;
     uint64_t tree_tiles = 0;  // all levels
     hipGraph_t graph = nullptr;
@@ -346,7 +348,7 @@ std::vector<DevBuf *> all_scratch(lbvh_ctx *ctx) {
           &ctx->tree_counts, &ctx->partials, &ctx->cen,
           &ctx->b_keys_a,
           &ctx->b_keys_b, &ctx->b_idx_a, &ctx->b_idx_b,  &ctx->b_digits,
-          &ctx->b_ord,    &ctx->b_bounds, &ctx->b_tree_items,
+          &ctx->b_bounds, &ctx->b_tree_items,
           &ctx->b_tree_counts, &ctx->b_table, &ctx->b_cen};
 }
 
@@ -782,22 +784,31 @@ int make_plan(lbvh_ctx *ctx, const uint32_t *offsets, uint32_t S) {
     return at;
   };
   P.o_seg_off = put(P.offsets);
-  std::vector<uint32_t> tile_seg, seg_tile0(S, 0);
+  std::vector<uint32_t> tile_seg, seg_tile0(S + 1, 0);
+  std::vector<uint32_t> blk_seg, seg_blk0(S + 1, 0);  // of the bounds
   std::vector<int> levels_k(S, 0);
   std::vector<std::vector<uint32_t>> grid_k(S);
   for (uint32_t k = 0; k < S; ++k) {
     const uint32_t n = offsets[k + 1] - offsets[k];
     seg_tile0[k] = (uint32_t)tile_seg.size();
-    for (uint32_t j = 0; j < batch_sort_tiles(n, P.items); ++j) tile_seg.push_back(k);
+    seg_blk0[k] = (uint32_t)blk_seg.size();
+    const uint32_t tiles = batch_sort_tiles(n, P.items);
+    tile_seg.insert(tile_seg.end(), tiles, k);
+    blk_seg.insert(blk_seg.end(), std::min(tiles, (uint32_t)kBoundsBlocks), k);
     if (n) {
       grid_k[k].resize(kMaxTreeLevels);
       levels_k[k] = tree_levels(n, P.tile, grid_k[k].data());
       P.levels = std::max(P.levels, levels_k[k]);
     }
   }
-  P.sort_tiles = (uint32_t)tile_seg.size();
-  P.o_tile_seg = put(tile_seg);
-  P.o_seg_tile0 = put(seg_tile0);
+  P.sort_tiles = seg_tile0[S] = (uint32_t)tile_seg.size();
+  P.bounds_blocks = seg_blk0[S] = (uint32_t)blk_seg.size();
+  P.o_tile_seg = P.o_blk_seg = put(tile_seg);
+  P.o_seg_tile0 = P.o_seg_blk0 = put(seg_tile0);
+  if (P.bounds_blocks != P.sort_tiles) {  // else a block per tile
+    P.o_blk_seg = put(blk_seg);
+    P.o_seg_blk0 = put(seg_blk0);
+  }
   // Tree levels: each mesh's tiles at level L are consecutive; a tile of
   // level L >= 1 reads the frontiers of its mesh's level L-1 tiles.
   std::vector<uint32_t> prev_tile0(S, 0), prev_tiles(S, 0);
@@ -832,14 +843,20 @@ void enqueue_batch(lbvh_ctx *ctx, const float *tri, bool have_bounds,
                    int32_t *perm) {
   const auto &P = ctx->plan;
   const uint32_t *T = static_cast<const uint32_t *>(ctx->b_table.ptr);
-  uint32_t *ord = static_cast<uint32_t *>(ctx->b_ord.ptr);
   const float4 *t4 = reinterpret_cast<const float4 *>(tri);
   const SortSegs ss{T + P.o_tile_seg, T + P.o_seg_tile0, T + P.o_seg_off,
                     P.items};
-  launch_batch_prologue(ord, P.S, !have_bounds, ctx->ctl, ctx->stream);
+  uint32_t *cnt = static_cast<uint32_t *>(ctx->b_digits.ptr);
+  uint32_t *off = cnt + (size_t)sort_radix(P.bits) * P.sort_tiles;
+  // the bounds lie where the offsets will be: a block's in a tile's
+  static_assert(64 <= 4 * kRadix, "a block's partial and fold, a tile's offsets");
+  float4 *partials = reinterpret_cast<float4 *>(off);
+  float4 *folded = partials + 2 * (size_t)P.bounds_blocks;
+  const BoundsBlocks bb{T + P.o_blk_seg, T + P.o_seg_blk0};
   float *cen = have_bounds ? nullptr : static_cast<float *>(ctx->b_cen.ptr);
   if (!have_bounds)
-    launch_batch_bounds(t4, ss, P.sort_tiles, ord, cen, P.total, ctx->stream);
+    launch_batch_bounds(t4, T + P.o_seg_off, bb, P.bounds_blocks, P.S,
+                        partials, folded, cen, P.total, ctx->stream);
   uint32_t *keys = static_cast<uint32_t *>(ctx->b_keys_a.ptr);
   uint32_t *tmp = static_cast<uint32_t *>(ctx->b_keys_b.ptr);
   uint32_t *out = skeys ? skeys : keys;
@@ -849,11 +866,8 @@ void enqueue_batch(lbvh_ctx *ctx, const float *tri, bool have_bounds,
   launch_batch_morton(t4, cen, P.total, ss, P.sort_tiles,
                       have_bounds ? static_cast<const float *>(ctx->b_bounds.ptr)
                                   : nullptr,
-                      ord, ctx->div_mode, keys,
-                      static_cast<uint32_t *>(ctx->b_digits.ptr), P.bits,
+                      bb, folded, ctx->div_mode, keys, cnt, P.bits,
                       ctx->stream);
-  uint32_t *cnt = static_cast<uint32_t *>(ctx->b_digits.ptr);
-  uint32_t *off = cnt + (size_t)sort_radix(P.bits) * P.sort_tiles;
   const SortPlan SP =
       sort_plan(P.bits, kKeyBits, keys, tmp, out, nullptr, vtmp, vout);
   for (int p = 0; p < SP.passes; ++p)
@@ -1507,7 +1521,6 @@ int lbvh_build_batched(lbvh_ctx *ctx, const float *tri,
   const uint64_t radix = sort_radix(P.bits);
   if ((st = ensure(ctx, ctx->b_digits, 8ull * radix * P.sort_tiles, false)))
     return st;
-  if ((st = ensure(ctx, ctx->b_ord, 32ull * num_meshes, false))) return st;
   if ((st = ensure(ctx, ctx->b_tree_items,
                    16ull * kItemInt4 * kTreeFrontier * P.tree_tiles, false)))
     return st;

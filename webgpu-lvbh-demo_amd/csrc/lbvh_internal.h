@@ -261,19 +261,25 @@ void launch_forest_level(int level, uint32_t grid, const float4 *tri,
                          Ctl *ctl, const TreeSegs &segs, hipStream_t s);
 
 // k_batch.hip
-void launch_batch_prologue(uint32_t *seg_ord, uint32_t num_segs,
-                           bool init_bounds, Ctl *ctl, hipStream_t s);
-// Per-mesh bounds (into seg_ord) and box centres (3 x total floats).
-void launch_batch_bounds(const float4 *tri, const SortSegs &segs,
-                         uint32_t tiles, uint32_t *seg_ord, float *cen,
-                         uint32_t total, hipStream_t s);
+// The blocks of a batch's bounds: each block's mesh, and each mesh's first block
+// (S + 1 entries).  A mesh has one per sort tile, at most kBoundsBlocks.
+struct BoundsBlocks {
+  const uint32_t *blk_seg;
+  const uint32_t *seg_blk0;
+};
+// Per-mesh bounds, two float4 each at the mesh's first block in `folded` (as
+// large as partials: two float4 a block), and box centres (3 x total floats).
+void launch_batch_bounds(const float4 *tri, const uint32_t *seg_off,
+                         const BoundsBlocks &blocks, uint32_t grid,
+                         uint32_t num_segs, float4 *partials, float4 *folded,
+                         float *cen, uint32_t total, hipStream_t s);
 // Per-mesh Morton keys and the first sort pass's per-tile digit counts;
 // centres from cen when non-null, else from tri.
 void launch_batch_morton(const float4 *tri, const float *cen, uint32_t total,
                          const SortSegs &segs, uint32_t tiles,
-                         const float *seg_bounds, const uint32_t *seg_ord,
-                         int div_mode, uint32_t *keys, uint32_t *cnt0,
-                         int bits, hipStream_t s);
+                         const float *seg_bounds, const BoundsBlocks &blocks,
+                         const float4 *folded, int div_mode, uint32_t *keys,
+                         uint32_t *cnt0, int bits, hipStream_t s);
 
 // k_raycast.hip
 void launch_raycast(const void *nodes, const float *tri, uint32_t n,
