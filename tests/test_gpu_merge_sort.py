@@ -49,3 +49,11 @@ def test_small_tiles(ctx, lb, ora, n):
     test_sort(ctx, n)
     for bounds in ("gpu", "caller"):
         test_build(ctx, lb, ora, n, bounds)
+
+
+# two rounds of 16: one tile past 8 and 16 groups, the largest build, the first
+# that takes radix passes
+@pytest.mark.parametrize("n", [65537, 262145, 300001, 393215, 393216, 393217])
+def test_two_rounds(ctx, lb, ora, n):
+    for bounds in ("gpu", "caller"):
+        test_build(ctx, lb, ora, n, bounds)

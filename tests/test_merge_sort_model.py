@@ -50,8 +50,9 @@ def merge_plan(n):
     """(run_log, log2 of the runs merged together) of each round."""
     runs, rounds, log = -(-n // TILE), [], TILE_LOG
     while runs > 1:
-        g = 3
+        g = 4
         if runs <= (16 if rounds else 32):
+            g = 3
             while 1 << g < runs:
                 g += 1
         rounds.append((log, g))

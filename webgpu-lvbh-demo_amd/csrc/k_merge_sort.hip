@@ -228,9 +228,11 @@ __device__ __forceinline__ bool sorts_below(uint32_t x, uint32_t k, bool le) {
   // without full keys a key plus one does not wrap
   return kFull ? (le ? x <= k : x < k) : x < k + (le ? 1u : 0u);
 }
-// One merge round: merges groups of kTpk * kPer runs of 2^run_log keys (the
-// last run and group may be short).  kTpk waves take 64 consecutive keys of a
-// run and kPer runs of its group each, and add their ranks up.
+// One merge round: merges groups of 4 kPer runs of 2^run_log keys (the last run
+// and group may be short).  A block's four waves take the same 64 consecutive
+// keys of a run and kPer runs of its group each, and add their ranks up.  (A
+// wave per 64 keys, for 8 runs, has its searches in a row: in the first of two
+// rounds over 33 tiles a build took 46.6 us, with four waves 42.0.)
 //
 // The ranks of the 64 keys in a run lie in a window that the first and the
 // last of them bound to within kSample keys: their ranks among the run's
@@ -257,31 +259,28 @@ __device__ __forceinline__ uint32_t count_below(uint32_t x, uint32_t k, bool le,
   return (uint32_t)__popcll(__ballot(sorts_below<kFull>(x, k, le)) & first);
 }
 
-template <int kTpk, int kPer, bool kFull>
+template <int kPer, bool kFull>
 __global__ __launch_bounds__(kMergeThreads) void k_merge(
     const uint32_t *__restrict__ keys_in, const int32_t *__restrict__ idx_in,
     const uint32_t *__restrict__ smp_in, uint32_t *__restrict__ keys_out,
     int32_t *__restrict__ idx_out, uint32_t *__restrict__ smp_out, uint32_t n,
     int run_log) {
-  constexpr uint32_t kRuns = kTpk * kPer;
-  constexpr int kChunks = kMergeWaves / kTpk;  // chunks of 64 keys per block
+  constexpr uint32_t kRuns = kMergeWaves * kPer;
   __shared__ uint32_t s_win[kMergeWaves][kPer * kWindow + (1 << kSteps) - kWindow];
   __shared__ uint32_t s_rank[kMergeWaves][64];
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t sub = wave % kTpk;
-  const uint32_t c0 =
-      (xcd_tile(blockIdx.x, gridDim.x) * kChunks + wave / kTpk) * 64;
+  const uint32_t c0 = xcd_tile(blockIdx.x, gridDim.x) * 64;
   const uint32_t i = c0 + lane;
   const uint32_t run = c0 >> run_log;  // the chunk's run: lengths are
   const uint32_t g0 = run & ~(kRuns - 1);  // multiples of 64
-  const uint32_t s0 = g0 + sub * kPer;     // this wave's runs
+  const uint32_t s0 = g0 + wave * kPer;    // this wave's runs
   uint32_t rank = 0, key = 0;
   int32_t val = 0;
   if (c0 < n) {
     const uint32_t at = min(i, n - 1);  // past the end: the last key again
     key = keys_in[at];
-    if (sub == 0) val = idx_in[at];
+    if (wave == 0) val = idx_in[at];
     // every 2^x-th sample: 64 per run (fewer of a run below 2^kMsTileLog)
     const int x = max(run_log - kMsTileLog, 0);
     const uint32_t have = n >> kSampleLog;
@@ -425,13 +424,11 @@ __global__ __launch_bounds__(kMergeThreads) void k_merge(
       for (int j = 0; j < kPer; ++j) rank += wide >> j & 1 ? p[j] - lo[j] : 0u;
     }
   }
-  if (kTpk > 1) {
-    s_rank[wave][lane] = rank;
-    __syncthreads();
-    if (sub != 0) return;
+  s_rank[wave][lane] = rank;
+  __syncthreads();
+  if (wave != 0) return;
 #pragma unroll
-    for (int g = 1; g < kTpk; ++g) rank += s_rank[wave + g][lane];
-  }
+  for (int g = 1; g < kMergeWaves; ++g) rank += s_rank[g][lane];
   if (i < n) {
     const uint32_t to = (g0 << run_log) + (i - (run << run_log)) + rank;
     if (to < n) {  // always, with sorted runs
@@ -455,9 +452,8 @@ static int tile_log(const MergeKeys &src, uint32_t n) {
   return n <= 8u << 9 ? 9 : n <= 16u << 10 ? 10 : kMsTileLog;
 }
 
-// The merge rounds of a sort of n keys: up to 32 tiles merge in one round,
-// four waves per 64 keys (their searches are the round's latency); more merge
-// 8 runs at a time, a wave per 64 keys, before a last round of up to 16.
+// The merge rounds of a sort of n keys: up to 32 tiles merge in one round; more
+// merge 16 runs at a time before a last round of up to 16.
 struct MergeRound {
   int run_log;          // runs of 2^run_log keys
   int group_log;        // 2^group_log of them merged together
@@ -467,9 +463,9 @@ static int merge_plan(const MergeKeys &src, uint32_t n, MergeRound *r) {
   int rounds = 0, log = tile_log(src, n);
   uint32_t runs = (n + (1u << log) - 1) >> log;
   while (runs > 1) {
-    int g = 3;
+    int g = 4;
     if (runs <= (rounds ? 16u : 32u))
-      while (1u << g < runs) ++g;
+      for (g = 3; 1u << g < runs;) ++g;
     r[rounds++] = {log, g};
     runs = (runs + (1u << g) - 1) >> g;
     log += g;
@@ -479,7 +475,7 @@ static int merge_plan(const MergeKeys &src, uint32_t n, MergeRound *r) {
 
 // Sample words of one buffer (merge_scratch_words holds two).
 static uint32_t merge_samples(uint32_t n) { return (n >> kSampleLog) + 1; }
-static_assert(kMergeSortMax <= 8u << kMaxRunLog, "the last round's runs");
+static_assert(kMergeBuildMax <= 16u << kMaxRunLog, "the last round's runs");
 static_assert(2 * ((kSmallSortTile >> kSampleLog) + 1) <= 2 * kRadix,
               "a radix sort's count words per tile hold its samples");
 
@@ -521,16 +517,13 @@ static void merge_rounds(const MergeKeys &src, uint32_t n, uint32_t *keys_tmp,
   int32_t *v = odd ? idx_tmp : idx_out, *v2 = odd ? idx_out : idx_tmp;
   for (int r = 0; r < count; ++r) {
     const int run_log = rounds[r].run_log, g = rounds[r].group_log;
-#define LBVH_MERGE(TPK, PER)                                                  \
-  hipLaunchKernelGGL((k_merge<TPK, PER, kFull>),                             \
-                     dim3((n + kMergeThreads / TPK - 1) /                    \
-                          (kMergeThreads / TPK)),                            \
+#define LBVH_MERGE(PER)                                                      \
+  hipLaunchKernelGGL((k_merge<PER, kFull>), dim3((n + 63) / 64),             \
                      dim3(kMergeThreads), 0, s, k, v, smp, k2, v2, smp2, n, \
                      run_log)
-    if (g == 5) LBVH_MERGE(4, 8);
-    else if (g == 4) LBVH_MERGE(4, 4);
-    else if (count == 1) LBVH_MERGE(4, 2);
-    else LBVH_MERGE(1, 8);
+    if (g == 5) LBVH_MERGE(8);
+    else if (g == 4) LBVH_MERGE(4);
+    else LBVH_MERGE(2);
 #undef LBVH_MERGE
     std::swap(k, k2);
     std::swap(v, v2);

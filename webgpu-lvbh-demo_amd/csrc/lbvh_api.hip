@@ -489,10 +489,10 @@ int bits_for(const lbvh_ctx *ctx, uint32_t n) {
                    untuned_bits(n));
 }
 
-// Whether a single-mesh sort of n keys merges sorted tiles; a fixed digit
-// width asks for the radix passes.
-bool merge_sorted(const lbvh_ctx *ctx, uint32_t n) {
-  return n <= kMergeSortMax && !(ctx->sort_bits_fixed && !ctx->tuning);
+// Whether a single-mesh sort of n keys (at most `most`) merges sorted tiles; a
+// fixed digit width asks for the radix passes.
+bool merge_sorted(const lbvh_ctx *ctx, uint32_t n, uint32_t most) {
+  return n <= most && !(ctx->sort_bits_fixed && !ctx->tuning);
 }
 
 // The key buffers of each pass of a sort from `in` to `out`: each pass reads
@@ -686,7 +686,7 @@ void build_pipeline(lbvh_ctx *ctx, const BuildScratch &S, const float *tri,
   const float4 *t4 = reinterpret_cast<const float4 *>(tri);
   uint32_t *skeys = sorted_keys_out ? sorted_keys_out : S.keys_a;
   int32_t *perm = perm_out ? perm_out : S.idx_a;
-  const bool merge = merge_sorted(ctx, n);
+  const bool merge = merge_sorted(ctx, n, kMergeBuildMax);
   // a mesh of one sort tile: the tile sort takes its bounds too
   const bool whole = merge && !bounds_host && n <= (uint32_t)kMsTile;
   MortonParams p{};
@@ -1316,7 +1316,7 @@ int lbvh_sort(lbvh_ctx *ctx, uint32_t *keys, int32_t *idx_out, uint32_t n) {
   // 10-bit digits take 4 passes here too, so they run only when fixed.
   const int bits = ctx->sort_bits_fixed ? ctx->sort_bits : kRadixBits;
   if ((st = ensure_sort_scratch(ctx, n, bits))) return st;
-  if (merge_sorted(ctx, n)) {
+  if (merge_sorted(ctx, n, kMergeSortMax)) {
     MergeKeys src{};
     src.keys = keys;
     uint32_t *kt = static_cast<uint32_t *>(ctx->keys_b.ptr);

@@ -166,15 +166,18 @@ void launch_single_key(const uint32_t *keys, uint32_t *sorted, int32_t *perm,
                        hipStream_t s);
 
 // k_merge_sort.hip
-// A single mesh of at most kMergeSortMax keys is sorted by tiles of kMsTile
-// keys in LDS and rank merges of the tiles, not by radix passes: one merge
-// round up to 32 tiles, two up to 128.  Builds of uniform meshes, merged
-// against the better digit width: 2^12 36 / 54 us, 2^16 47 / 67, 2^17 65 / 81,
-// 2^18 81 / 93 (heightfields: 38 / 56, 52 / 68, 71 / 79, 84 / 90); a third
-// round loses to the radix passes (300,000: 111 / 105).
+// A sort of at most kMergeSortMax keys, or a build's of at most kMergeBuildMax,
+// goes by tiles of up to kMsTile keys in LDS and rank merges of the tiles, not
+// by radix passes: one merge round up to 32 tiles, two beyond.  A build saves
+// its Morton launch too, so its line lies higher.  Builds of uniform meshes in
+// us, merged / by the better digit width: 66,000 41.8 / 60.9, 2^17 48.1 / 65.5,
+// 2^18 63.7 / 79.8, 300,000 75.5 / 87.0, 393,216 87.2 / 96.2 (heightfields 43.6 /
+// 60.3, 50.3 / 63.7, 63.3 / 75.3, 77.7 / 85.9, 90.1 / 93.0), 2^19 107.9 / 104.9;
+// sorts of random keys 66,000 23.0 / 45.5, 2^18 35.7 / 46.3, 280,000 49.1 / 47.6.
 constexpr int kMsTileLog = 11;
 constexpr int kMsTile = 1 << kMsTileLog;
 constexpr uint32_t kMergeSortMax = 128u << kMsTileLog;
+constexpr uint32_t kMergeBuildMax = 192u << kMsTileLog;
 // The keys of a merge sort: given (any u32; `keys` may be the output), or
 // Morton keys made by the tile sort -- from the centres launch_bounds wrote
 // with the bounds folded from its `parts` partials, from the triangles with the bounds in p, or (whole: n <= kMsTile) from the triangles
