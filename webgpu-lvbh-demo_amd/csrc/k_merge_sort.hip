@@ -15,7 +15,7 @@
 //                  its rank in each other run of its group and moves there
 //                  (7 us for 32 runs of 2,048).
 // Ranks cost (runs - 1) searches per key, so it pays while the chip is far
-// from full (kMergeSortMax).
+// from full (kMergeSortMax, kMergeBuildMax).
 #include <algorithm>
 #include <utility>
 
@@ -228,11 +228,10 @@ __device__ __forceinline__ bool sorts_below(uint32_t x, uint32_t k, bool le) {
   // without full keys a key plus one does not wrap
   return kFull ? (le ? x <= k : x < k) : x < k + (le ? 1u : 0u);
 }
-// One merge round: merges groups of 4 kPer runs of 2^run_log keys (the last run
-// and group may be short).  A block's four waves take the same 64 consecutive
-// keys of a run and kPer runs of its group each, and add their ranks up.  (A
-// wave per 64 keys, for 8 runs, has its searches in a row: in the first of two
-// rounds over 33 tiles a build took 46.6 us, with four waves 42.0.)
+// One merge round: merges groups of kWaves x kPer runs of 2^run_log keys (the
+// last run and group may be short).  A block's waves take the same 64
+// consecutive keys of a run and kPer runs of its group each, and add their
+// ranks up.
 //
 // The ranks of the 64 keys in a run lie in a window that the first and the
 // last of them bound to within kSample keys: their ranks among the run's
@@ -243,8 +242,6 @@ __device__ __forceinline__ bool sorts_below(uint32_t x, uint32_t k, bool le) {
 // windows of exact size, searched in fewer but computed steps, took twice as
 // long, as did whole tiles in LDS (L2 bandwidth).  Wider windows, where the
 // runs' keys are spread unevenly, are searched in place.
-constexpr int kMergeThreads = 256;
-constexpr int kMergeWaves = kMergeThreads / 64;
 // Between evenly spread runs a window holds 64 + 31 keys on average, with a
 // deviation near 17: at 128 a fifth of the waves of 8 runs met a wider one.
 constexpr int kWindow = 192;
@@ -259,15 +256,15 @@ __device__ __forceinline__ uint32_t count_below(uint32_t x, uint32_t k, bool le,
   return (uint32_t)__popcll(__ballot(sorts_below<kFull>(x, k, le)) & first);
 }
 
-template <int kPer, bool kFull>
-__global__ __launch_bounds__(kMergeThreads) void k_merge(
+template <int kWaves, int kPer, bool kFull>
+__global__ __launch_bounds__(64 * kWaves) void k_merge(
     const uint32_t *__restrict__ keys_in, const int32_t *__restrict__ idx_in,
     const uint32_t *__restrict__ smp_in, uint32_t *__restrict__ keys_out,
     int32_t *__restrict__ idx_out, uint32_t *__restrict__ smp_out, uint32_t n,
     int run_log) {
-  constexpr uint32_t kRuns = kMergeWaves * kPer;
-  __shared__ uint32_t s_win[kMergeWaves][kPer * kWindow + (1 << kSteps) - kWindow];
-  __shared__ uint32_t s_rank[kMergeWaves][64];
+  constexpr uint32_t kRuns = kWaves * kPer;
+  __shared__ uint32_t s_win[kWaves][kPer * kWindow + (1 << kSteps) - kWindow];
+  __shared__ uint32_t s_rank[kWaves][64];
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t c0 = xcd_tile(blockIdx.x, gridDim.x) * 64;
@@ -428,7 +425,7 @@ __global__ __launch_bounds__(kMergeThreads) void k_merge(
   __syncthreads();
   if (wave != 0) return;
 #pragma unroll
-  for (int g = 1; g < kMergeWaves; ++g) rank += s_rank[g][lane];
+  for (int g = 1; g < kWaves; ++g) rank += s_rank[g][lane];
   if (i < n) {
     const uint32_t to = (g0 << run_log) + (i - (run << run_log)) + rank;
     if (to < n) {  // always, with sorted runs
@@ -452,8 +449,12 @@ static int tile_log(const MergeKeys &src, uint32_t n) {
   return n <= 8u << 9 ? 9 : n <= 16u << 10 ? 10 : kMsTileLog;
 }
 
-// The merge rounds of a sort of n keys: up to 32 tiles merge in one round; more
-// merge 16 runs at a time before a last round of up to 16.
+// The merge rounds of a sort of n keys: up to 32 tiles merge in one round, eight
+// waves per 64 keys, since their searches in a row are its time (builds of
+// 50,000 39.4 us with four waves, 37.7 with eight; heightfields 40.3, 38.1).
+// More tiles merge 16 runs at a time, four waves (with one, for 8 runs, 66,000
+// triangles took 46.6 us, with four 42.0), before a last round of up to 16; with
+// eight waves 2^18 triangles take 66.5 us, not 63.4.
 struct MergeRound {
   int run_log;          // runs of 2^run_log keys
   int group_log;        // 2^group_log of them merged together
@@ -517,13 +518,18 @@ static void merge_rounds(const MergeKeys &src, uint32_t n, uint32_t *keys_tmp,
   int32_t *v = odd ? idx_tmp : idx_out, *v2 = odd ? idx_out : idx_tmp;
   for (int r = 0; r < count; ++r) {
     const int run_log = rounds[r].run_log, g = rounds[r].group_log;
-#define LBVH_MERGE(PER)                                                      \
-  hipLaunchKernelGGL((k_merge<PER, kFull>), dim3((n + 63) / 64),             \
-                     dim3(kMergeThreads), 0, s, k, v, smp, k2, v2, smp2, n, \
+#define LBVH_MERGE(WAVES, PER)                                            \
+  hipLaunchKernelGGL((k_merge<WAVES, PER, kFull>), dim3((n + 63) / 64),   \
+                     dim3(64 * WAVES), 0, s, k, v, smp, k2, v2, smp2, n, \
                      run_log)
-    if (g == 5) LBVH_MERGE(8);
-    else if (g == 4) LBVH_MERGE(4);
-    else LBVH_MERGE(2);
+    if (count == 1) {
+      if (g == 5) LBVH_MERGE(8, 4);
+      else if (g == 4) LBVH_MERGE(8, 2);
+      else LBVH_MERGE(8, 1);
+    } else {
+      if (g == 4) LBVH_MERGE(4, 4);
+      else LBVH_MERGE(4, 2);
+    }
 #undef LBVH_MERGE
     std::swap(k, k2);
     std::swap(v, v2);
