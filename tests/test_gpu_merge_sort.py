@@ -44,7 +44,7 @@ def test_build(ctx, lb, ora, n, bounds):
 
 
 # where the tile grows: one tile of 512, 1,024 or 2,048 keys, then several
-@pytest.mark.parametrize("n", [511, 512, 513, 1023, 1024, 1025, 1537, 3000, 4096, 4097, 8193, 16383])
+@pytest.mark.parametrize("n", [511, 512, 513, 1023, 1024, 1025, 1537, 3000, 4096, 4097, 8192, 8193, 16383, 32768])
 def test_small_tiles(ctx, lb, ora, n):
     test_sort(ctx, n)
     for bounds in ("gpu", "caller"):

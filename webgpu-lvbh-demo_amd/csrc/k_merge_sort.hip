@@ -438,15 +438,16 @@ __global__ __launch_bounds__(64 * kWaves) void k_merge(
 
 // Keys per tile, 2^this.  A block's rounds take 10-11 us at 2,048 keys, 16
 // waves on one CU, and less with fewer on more CUs, while the merge of all the
-// tiles stays one round of a few runs.  Builds in us by tile of 2,048 / 1,024 /
-// 512 keys: 2,500 triangles 26.3 / 23.4 / 22.0, 5,000 26.9 / 23.3 / 23.1
-// (heightfield 27.1 / 24.3 / 24.7), 16,384 31.1 / 28.7 / 28.8 (31.9 / 30.5 /
-// 32.1); heightfields of 20,000 turn, 34.0 / 34.5 / 34.8.  One tile needs no
-// merge: 1,024 triangles with caller bounds 16.2 / 15.4 / 17.7.
+// tiles stays one round.  Builds in us by tile of 2,048 / 1,024 / 512 keys:
+// 2,500 triangles 26.3 / 23.4 / 22.1, 8,192 (caller bounds) - / 20.4 / 19.7,
+// 16,384 31.1 / 28.3 / 28.8, 20,000 32.7 / 31.2 (heightfields 32.6 / 32.1), 32,768
+// 33.1 / 31.4 (33.6 / 33.4); 64 tiles of 1,024 in one round turn, 65,536 37.2 /
+// 38.3 (39.8 / 45.5).  One tile needs no merge: 1,024 triangles with caller bounds
+// 16.2 / 15.4 / 17.7.
 static int tile_log(const MergeKeys &src, uint32_t n) {
   if (n <= 1u << 10) return n <= 1u << 9 ? 9 : 10;
   if (src.whole) return kMsTileLog;
-  return n <= 8u << 9 ? 9 : n <= 16u << 10 ? 10 : kMsTileLog;
+  return n <= 16u << 9 ? 9 : n <= 32u << 10 ? 10 : kMsTileLog;
 }
 
 // The merge rounds of a sort of n keys: up to 32 tiles merge in one round, eight
