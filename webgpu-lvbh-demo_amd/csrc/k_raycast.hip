@@ -88,8 +88,9 @@ constexpr uint32_t kRayChunk = 64;  // consecutive blocks on one XCD
 //   * kRayChunk blocks (4,096 rays) in a row run on one XCD, whose L2 then
 //     holds the nodes they share (1M rays of a frame over 1M triangles 398 ->
 //     317 us).
-// Together 245 -> 181 us for a 512 x 512 frame over 100,000 clustered
-// triangles, 1,000 -> 740 us for 1M scattered rays over 1M.  Dropping popped
+//   * the stack's top is at hand when a step ends in a pop.
+// Together 245 -> 172 us for a 512 x 512 frame over 100,000 clustered
+// triangles (186 before the last), 1,000 -> 740 us for 1M scattered rays over 1M.  Dropping popped
 // nodes beyond the closest hit lost (the stack entries double), and so did
 // descending to a leaf per lane before any test, and touching both children
 // ahead.
@@ -127,6 +128,10 @@ __global__ __launch_bounds__(kRayThreads) void k_raycast(
     const int4 *at = leaf ? tri + 3 * (size_t)(id < n ? id : 0u)
                           : nodes + 4 * (size_t)id;
     const int4 a = at[0], b = at[1], c = at[2], e = at[leaf ? 2 : 3];
+    // The stack's top, read from LDS while those loads are under way.  (Read
+    // when it is popped, from LDS or scratch by its depth, it was one generic
+    // load, which waits on the vector memory path.)
+    int top = s_stack[min(max(sp - 1, 0), kRayLds - 1)][tid];
     bool next;  // the next node comes off the stack
     if (leaf) {
       const float h = tri_distance(o, d, v3(a), v3(b), v3(c));
@@ -152,8 +157,8 @@ __global__ __launch_bounds__(kRayThreads) void k_raycast(
     }
     if (next) {
       sp -= 1;
-      if (sp >= 0)
-        node = sp < kRayLds ? s_stack[sp][tid] : deep[sp - kRayLds];
+      if (sp >= kRayLds) top = deep[sp - kRayLds];
+      node = top;
     }
   }
   // RayHit: normal facing the ray, dist -1 for a miss (pathtracer.js:572-583)
