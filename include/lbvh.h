@@ -96,7 +96,8 @@ int lbvh_get_div_mode(const lbvh_ctx *ctx);
 typedef enum {
   LBVH_TUNE_TREE_TILE = 0, /* leaves per block of the fused up pass:
                               256|512|1024.  Not fixed, builds and refits of
-                              at most 2^23 triangles take tiles of their own
+                              at most 3,670,016 triangles take tiles of
+                              their own
                               (256 leaves, no climb) */
   LBVH_TUNE_SORT_BITS = 1  /* digit width of the builds' radix sort: 8 (4
                               passes over the 30-bit Morton keys) or 10 (3

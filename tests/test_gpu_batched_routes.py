@@ -1,6 +1,6 @@
-"""The routes of a batched build: sort tiles of 1,024 keys and k_forest.hip's
-tree levels up to 2^23 triangles in all, larger tiles and k_tree.hip's past it
-or under an HBM budget; meshes that begin at any offset, whole and part tiles."""
+"""The routes of a batched build: sort tiles of 1,024 keys up to 2^23 triangles
+in all and k_forest.hip's leaf tiles up to 7 * 2^19, larger tiles and k_tree.hip's
+past them or under an HBM budget; meshes that begin at any offset, whole and part tiles."""
 import numpy as np
 import pytest
 
@@ -9,6 +9,7 @@ from test_gpu_batched import make_batch, run_batch
 pytestmark = pytest.mark.gpu
 
 SMALL = [1, 1023, 1024, 1025, 3, 4096, 4097, 4095, 255, 257, 16385, 2, 70001]
+MIDDLE = SMALL + [262144, 131073, 100003] * 7  # 3.6M
 LARGE = SMALL + [262144, 131073, 100003] * 16  # 7.9M
 # meshes of more sort tiles than bounds blocks, and empty ones
 FEW = [3, 600001, 0, 0, 1030, 524289, 0, 7] + [0] * 300 + [2]
@@ -17,7 +18,7 @@ LARGER = LARGE + [262144, 262143]              # past 2^23
 
 @pytest.mark.parametrize("bits", [8, 10])
 @pytest.mark.parametrize("with_bounds", [False, True])
-@pytest.mark.parametrize("sizes", [SMALL, FEW, LARGE, LARGER], ids=["small", "few", "large", "larger"])
+@pytest.mark.parametrize("sizes", [SMALL, FEW, MIDDLE, LARGE, LARGER], ids=["small", "few", "middle", "large", "larger"])
 def test_routes_agree(lb, ora, sizes, with_bounds, bits):
     meshes, offsets, tri = make_batch(lb, sizes, 300)
     bounds = None

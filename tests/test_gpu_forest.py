@@ -34,7 +34,7 @@ def test_build_and_refit(ctx, lb, ora, n):
                 b.destroy()
 
 
-@pytest.mark.parametrize("n", [300, 100000, 1 << 23, (1 << 23) + 1])
+@pytest.mark.parametrize("n", [300, 100000, 7 << 19, (7 << 19) + 1, 1 << 23, (1 << 23) + 1])
 def test_routes_agree(lb, n):
     """Free, under a budget (which takes the larger leaf tile) and with the
     tile fixed: the same words, up to the largest mesh and past it."""

@@ -11,7 +11,7 @@
 //     and builds the Karras tree bottom-up (Apetrei 2014) without a parents
 //     array, merging inside LDS wherever both children of a split lie in
 //     the block's tile; each tile passes the subtrees it cannot complete
-//     (its frontier) to k_items, whose levels merge the frontiers of 32
+//     (its frontier) to the item levels, which merge the frontiers of 32
 //     tiles per block until one block completes the root.
 //
 // Common definitions.  Sorted position i, key k_i.  delta(i, j) = common
@@ -894,14 +894,12 @@ __global__ __launch_bounds__(kMapThreads) void k_rearrange(
 // range's two boundary gaps) into the tile's own kFrontierMax slots, with
 // their count.
 //
-// Level L >= 1 builds the tree over items: one block of kItemTile threads
-// takes the frontiers of fan_in(...) consecutive tiles of level L-1, in rounds
-// of at most kItemTile items (the previous round's frontier, then the next
-// source items), until a single tile holds all of a mesh's remaining items
-// and completes its root.  Frontier items are the subtrees hanging off
-// root paths, so climbing over them would be a serial chain of merges as
-// long as those paths; the item levels compute their nodes in parallel
-// instead (k_items).  The level plan depends only on
+// Level L >= 1 builds the tree over items, the frontiers of fan_in(...)
+// consecutive tiles of level L-1 a block, until a single tile holds all of a
+// mesh's remaining items and completes its root.  Frontier items are the
+// subtrees hanging off root paths, so climbing over them would be a serial
+// chain of merges as long as those paths; the item levels compute their nodes
+// in parallel instead (k_forest.hip).  The level plan depends only on
 // the leaf count, so no block waits for another and no counter is shared.
 // (A dynamic tile ticket -- one same-address device-scope atomic per tile --
 // and a look-back across tiles both serialise on MI355X, where those
@@ -909,12 +907,7 @@ __global__ __launch_bounds__(kMapThreads) void k_rearrange(
 // the stage time.)  Nodes are written exactly once, by the thread that
 // merges their children, as soon as their Karras id is known.
 
-constexpr int kItemTile = 1024;
-static_assert(kFanIn <= kFanInMax && kFanInMax < kItemTile &&
-                  (kFanInMax & (kFanInMax - 1)) == 0,
-              "one thread per source tile; binary search over them");
-
-// Frontier output shared by both level kinds: the stopped subtrees that
+// Frontier output: the stopped subtrees that
 // leave the tile, in item order, into the tile's kFrontierMax slots.  An item
 // is its leaf range, its box and the deltas at the gaps on either side of
 // the range, so the level above needs no sorted keys.  Returns the count
@@ -1142,281 +1135,6 @@ __global__ __launch_bounds__(T) void k_leaves(
                 items_out, count_out, ctl, tid, T);
 }
 
-// ---- levels >= 1: items ---------------------------------------------------
-
-// One item level: tile = the frontiers of fan_in consecutive tiles of the
-// level below.  Level L-1's tile g keeps its items in
-// items_in[g * kFrontierMax ...] and their number in count_in[g].
-//
-// The block sweeps them in rounds of m <= kItemTile items: the frontier the
-// previous round emitted (read back from the tile's own output slots; it is
-// the frontier of every leaf so far, at most kFrontierMax items) followed by
-// as many of the next source items as fit.  A round's last gap carries the
-// delta to the next round's first leaf, so the nodes it cannot complete
-// stay roots, exactly as at the block's own edge.  Typical frontiers are
-// small, and a level usually takes a single round.
-//
-// The tree over the block's m items is the min-Cartesian tree of the deltas
-// at the gaps between them: the node split at gap g spans, on each side, up
-// to the nearest gap with a smaller delta (equal deltas never face each
-// other across a larger-delta stretch, so "smaller" is unambiguous); gap -1
-// before the first item and gap m-1 after the last one carry the deltas to
-// the leaves outside the block.  A node is complete, and written here, when
-// both bounds are found; its parent is the bound with the larger delta.
-// So, with one thread per gap and O(log m) LDS steps each instead of a serial
-// climb:
-//   1. load the items; the gap deltas form a sparse table of range minima
-//      (position p = gap + 1) and the item boxes a segment tree;
-//   2. each gap finds its nearest smaller delta on either side by binary
-//      lifting over the table; a complete node takes its children's boxes
-//      from the segment tree and is written at its Karras id;
-//   3. the roots of the resulting forest -- complete nodes and items whose
-//      parent gap is incomplete or outside the block -- are the frontier,
-//      marked at their first item so the emit keeps leaf order.
-constexpr int kItemLog = 10;
-static_assert(kItemTile == 1 << kItemLog, "sparse table levels");
-
-struct ItemLds {
-  signed char dm[kItemLog + 1][kItemTile + 2];  // range minima of gap deltas
-  float smn[3][2 * kItemTile], smx[3][2 * kItemTile];  // box segment tree
-  int il[kItemTile], ir[kItemTile];  // leaf range of each item
-  short qL[kItemTile], qR[kItemTile];  // per gap: nearest smaller positions
-  unsigned char complete[kItemTile];  // per gap: node complete in the block
-  int root_of[kItemTile];  // per first item: frontier root (gap, T + item)
-  uint32_t wsum[16];
-  uint32_t pre[kFanInMax + 1];  // first item of each source tile
-};
-
-// Box of items [a, b] from the segment tree (leaves at kItemTile + item).
-__device__ __forceinline__ void item_range_box(const ItemLds &L, int a, int b,
-                                               float mn[3], float mx[3]) {
-  mn[0] = mn[1] = mn[2] = INFINITY;
-  mx[0] = mx[1] = mx[2] = -INFINITY;
-  int lo = a + kItemTile, hi = b + kItemTile + 1;
-  while (lo < hi) {
-    if (lo & 1) {
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        mn[c] = qmin(mn[c], L.smn[c][lo]);
-        mx[c] = qmax(mx[c], L.smx[c][lo]);
-      }
-      ++lo;
-    }
-    if (hi & 1) {
-      --hi;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        mn[c] = qmin(mn[c], L.smn[c][hi]);
-        mx[c] = qmax(mx[c], L.smx[c][hi]);
-      }
-    }
-    lo >>= 1;
-    hi >>= 1;
-  }
-}
-
-// One round of k_items over m items: items [0, carry) are the tile's own
-// output slots (the previous round's frontier), items [carry, m) the source
-// items from `taken` on.  Writes the nodes it completes and leaves the
-// forest roots in L.root_of (gap, or kItemTile + item) with L.qL / L.qR.
-__device__ __forceinline__ void item_round(ItemLds &L, int m, int carry,
-                                           int taken, uint32_t src0,
-                                           const int4 *__restrict__ items_in,
-                                           const int4 *items_out,
-                                           uint32_t gtile, uint32_t N,
-                                           int4 *nodes) {
-  constexpr int T = kItemTile;
-  const int tid = threadIdx.x;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    L.smn[c][T + tid] = INFINITY;  // leaves past the items stay neutral
-    L.smx[c][T + tid] = -INFINITY;
-  }
-  L.complete[tid] = 0;
-  L.root_of[tid] = -1;
-  __syncthreads();
-
-  // 1. items: leaf ranges, boxes (segment-tree leaves), gap deltas
-  if (tid < m) {
-    const int4 *src;
-    if (tid < carry) {
-      src = items_out + kItemInt4 * ((size_t)gtile * kFrontierMax + tid);
-    } else {
-      // the source tile holding item g: the last s with pre[s] <= g
-      const int g = taken + tid - carry;
-      int s = 0;
-#pragma unroll
-      for (int step = kFanInMax / 2; step > 0; step >>= 1)
-        if ((int)L.pre[s + step] <= g) s += step;
-      src = items_in + kItemInt4 * ((size_t)(src0 + s) * kFrontierMax +
-                                    (uint32_t)(g - (int)L.pre[s]));
-    }
-    const int4 a = src[0], b = src[1], g = src[2];
-    L.il[tid] = a.x;
-    L.ir[tid] = a.y;
-    L.smn[0][T + tid] = __int_as_float(a.z);
-    L.smn[1][T + tid] = __int_as_float(a.w);
-    L.smn[2][T + tid] = __int_as_float(b.x);
-    L.smx[0][T + tid] = __int_as_float(b.y);
-    L.smx[1][T + tid] = __int_as_float(b.z);
-    L.smx[2][T + tid] = __int_as_float(b.w);
-    L.dm[0][tid + 1] = (signed char)g.y;  // delta at the gap after the item
-    if (tid == 0) L.dm[0][0] = (signed char)g.x;  // and before the first one
-  }
-  __syncthreads();
-  // Table and tree levels for m items: lifting over levels 0..L reaches
-  // 2^(L+1) - 1 positions (>= m - 1 needed), and a range query reads tree
-  // nodes no larger than its m leaves.  m <= 1024 keeps L <= kItemLog.
-  const int levels = min(32 - __clz((uint32_t)m), kItemLog);
-  for (int lv = 1; lv <= levels; ++lv) {
-    const int w = 1 << lv;
-    // range minima over positions [p, p + w) for p + w <= m + 1
-    if (tid + w <= m + 1)
-      L.dm[lv][tid] = min(L.dm[lv - 1][tid], L.dm[lv - 1][tid + (w >> 1)]);
-    if (tid < (T >> lv)) {
-      const int i = (T >> lv) + tid;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        L.smn[c][i] = qmin(L.smn[c][2 * i], L.smn[c][2 * i + 1]);
-        L.smx[c][i] = qmax(L.smx[c][2 * i], L.smx[c][2 * i + 1]);
-      }
-    }
-    __syncthreads();
-  }
-
-  // 2. gap tid: its node's extent, and the node when complete
-  if (tid < m - 1) {
-    const int p = tid + 1;
-    const int d = L.dm[0][p];
-    // binary lifting on both sides at once (two independent LDS chains):
-    // [cl, p) and (p, cr) hold no delta below d
-    int cl = p, cr = p + 1;
-    for (int lv = levels; lv >= 0; --lv) {
-      const int w = 1 << lv;
-      const bool gl = cl - w >= 0 && L.dm[lv][cl - w] >= d;
-      const bool gr = cr + w - 1 <= m && L.dm[lv][cr] >= d;
-      if (gl) cl -= w;
-      if (gr) cr += w;
-    }
-    const int qL = cl - 1;  // -1: none inside the block
-    const int qR = cr <= m ? cr : -1;
-    L.qL[tid] = (short)qL;
-    L.qR[tid] = (short)qR;
-    if (qL >= 0 && qR >= 0) {
-      L.complete[tid] = 1;
-      const int a = qL, b = qR - 1;  // the node's first and last item
-      float lmn[3], lmx[3], rmn[3], rmx[3];
-      item_range_box(L, a, tid, lmn, lmx);
-      item_range_box(L, tid + 1, b, rmn, rmx);
-      const int Lr = L.il[a], s = L.ir[tid], Rr = L.ir[b];
-      const int dl = L.dm[0][qL], dr = L.dm[0][qR];
-      const bool root = (Lr == 0 && Rr == (int)N - 1);
-      const int K = root ? 0 : (dr > dl ? Rr : Lr);
-      const int lid = (Lr == s) ? -(s + 1) : s;
-      const int rid = (Rr == s + 1) ? -(s + 2) : s + 1;
-      int4 *node = nodes + 4 * (size_t)K;
-      node[0] = pack3(lmn, lid);
-      node[1] = pack3(lmx, 2);
-      node[2] = pack3(rmn, rid);
-      node[3] = pack3(rmx, 0);
-    }
-  }
-  __syncthreads();
-
-  // 3. roots of the forest, marked at their first item
-  if (tid < m - 1 && L.complete[tid]) {
-    const int qL = L.qL[tid], qR = L.qR[tid];
-    const int a = qL, b = qR - 1;
-    if (!(L.il[a] == 0 && L.ir[b] == (int)N - 1)) {  // the mesh root has none
-      const int parent = L.dm[0][qR] > L.dm[0][qL] ? qR - 1 : qL - 1;
-      if (!(parent >= 0 && parent <= m - 2 && L.complete[parent]))
-        L.root_of[a] = tid;
-    }
-  }
-  if (tid < m && !(L.il[tid] == 0 && L.ir[tid] == (int)N - 1)) {
-    const int parent = L.dm[0][tid + 1] > L.dm[0][tid] ? tid : tid - 1;
-    if (!(parent >= 0 && parent <= m - 2 && L.complete[parent]))
-      L.root_of[tid] = T + tid;
-  }
-  __syncthreads();
-}
-
-__global__ __launch_bounds__(kItemTile) void k_items(
-    uint32_t n_all,
-    const int4 *__restrict__ items_in, const uint32_t *__restrict__ count_in,
-    uint32_t prev_tiles_all, int4 *items_out,  // written, then read back
-    uint32_t *__restrict__ count_out, int4 *nodes_all, Ctl *ctl,
-    TreeSegs segs) {
-  constexpr int T = kItemTile;
-  __shared__ ItemLds L;
-  const int tid = threadIdx.x;
-  const uint32_t gtile = xcd_tile(blockIdx.x, gridDim.x);
-  uint32_t tile0 = 0, leaf_base = 0, N = n_all, prev0 = 0,
-           prev_tiles = prev_tiles_all;
-  if (segs.tile_seg) {
-    const uint32_t sg = segs.tile_seg[gtile];
-    tile0 = segs.seg_tile0[sg];
-    leaf_base = segs.seg_off[sg];
-    N = segs.seg_off[sg + 1] - leaf_base;
-    prev0 = segs.prev_tile0[sg];
-    prev_tiles = segs.prev_tiles[sg];
-  }
-  const uint32_t tile = gtile - tile0;  // tile within the mesh
-  int4 *nodes = nodes_all + 4 * (size_t)leaf_base;
-  const uint32_t fan = fan_in(prev_tiles);
-  const uint32_t src0 = prev0 + tile * fan;  // first source tile
-  {
-    // item prefix over the source tiles: L.pre[s] = first item of tile s
-    // (the total from s = nsrc on)
-    const uint32_t first = tile * fan;
-    const uint32_t nsrc =
-        prev_tiles > first ? min(fan, prev_tiles - first) : 0u;
-    const uint32_t c = (uint32_t)tid < nsrc
-                           ? min(count_in[src0 + tid], (uint32_t)kFrontierMax)
-                           : 0u;
-    const uint32_t ex = block_exclusive_scan(c, L.wsum);
-    if (tid <= kFanInMax) L.pre[tid] = ex;
-  }
-  __syncthreads();
-  const int total = (int)L.pre[kFanInMax];
-  int taken = 0;  // source items used by earlier rounds
-  int carry = 0;  // items of the previous round's frontier
-  while (true) {
-    const int fresh = min(total - taken, T - carry);
-    const bool last = taken + fresh == total;
-    const int m = carry + fresh;
-    item_round(L, m, carry, taken, src0, items_in, items_out, gtile, N,
-               nodes);
-    // the round's frontier: the next round's first items, or the output
-    const int v = tid < m ? L.root_of[tid] : -1;
-    const bool out = v >= 0;
-    int fl = 0, fr = 0, fdl = 0, fdr = 0;
-    float fmn[3] = {0.f, 0.f, 0.f}, fmx[3] = {0.f, 0.f, 0.f};
-    if (out) {
-      int a, b;
-      if (v >= T) {
-        a = b = v - T;
-      } else {
-        a = L.qL[v];
-        b = L.qR[v] - 1;
-      }
-      item_range_box(L, a, b, fmn, fmx);
-      fl = L.il[a];
-      fr = L.ir[b];
-      fdl = L.dm[0][a];
-      fdr = L.dm[0][b + 1];
-    }
-    __syncthreads();  // every read of this round's items is done
-    const uint32_t count = emit_frontier(out, fl, fr, fdl, fdr, fmn, fmx,
-                                         L.wsum, gtile, items_out, count_out,
-                                         ctl, tid, T);
-    if (last) break;
-    taken += fresh;
-    carry = (int)min(count, (uint32_t)kFrontierMax);
-    __syncthreads();  // the emitted items are visible to the whole block
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
@@ -1551,21 +1269,14 @@ static void launch_leaf_level(uint32_t grid, const int4 *t4,
                      n, o4, items_out, count_out, n4, ctl, segs);
 }
 
-void launch_tree_level(int level, int tile, uint32_t grid, const float4 *tri,
-                       const uint32_t *skeys, const int32_t *perm, uint32_t n,
-                       float4 *otri, const int4 *items_in,
-                       const uint32_t *count_in, uint32_t prev_tiles,
-                       int4 *items_out, uint32_t *count_out, float4 *nodes,
-                       Ctl *ctl, const TreeSegs &segs, hipStream_t s) {
+void launch_leaves(int tile, uint32_t grid, const float4 *tri,
+                   const uint32_t *skeys, const int32_t *perm, uint32_t n,
+                   float4 *otri, int4 *items_out, uint32_t *count_out,
+                   float4 *nodes, Ctl *ctl, const TreeSegs &segs,
+                   hipStream_t s) {
   const int4 *t4 = reinterpret_cast<const int4 *>(tri);
   int4 *o4 = reinterpret_cast<int4 *>(otri);
   int4 *n4 = reinterpret_cast<int4 *>(nodes);
-  if (level > 0) {
-    hipLaunchKernelGGL(k_items, dim3(grid), dim3(kItemTile), 0, s, n,
-                       items_in, count_in, prev_tiles, items_out, count_out,
-                       n4, ctl, segs);
-    return;
-  }
   switch (tile) {
     case 256:
       launch_leaf_level<256>(grid, t4, skeys, perm, n, o4, items_out,

@@ -586,15 +586,15 @@ void run_tree(lbvh_ctx *ctx, int4 *items, uint32_t *counts, const float *tri,
     StageScope sc(ctx, L ? LBVH_STAGE_TREE_TOP : LBVH_STAGE_TREE);
     const int4 *items_in = items + kItemInt4 * kTreeFrontier * prev;
     int4 *items_out = items + kItemInt4 * kTreeFrontier * base;
-    const uint32_t below = L ? grid[L - 1] : 0u;
-    if (plan.forest)
-      launch_forest_level(L, grid[L], t4, skeys, perm, n, o4, items_in,
-                          counts + prev, below, items_out, counts + base,
-                          nodes, ctx->ctl, TreeSegs{}, ctx->stream);
+    if (L)
+      launch_items(grid[L], n, items_in, counts + prev, grid[L - 1], items_out,
+                   counts + base, nodes, ctx->ctl, TreeSegs{}, ctx->stream);
+    else if (plan.forest)
+      launch_forest_leaves(grid[0], t4, skeys, perm, n, o4, items_out, counts,
+                           nodes, ctx->ctl, TreeSegs{}, ctx->stream);
     else
-      launch_tree_level(L, plan.tile, grid[L], t4, skeys, perm, n, o4, items_in,
-                        counts + prev, below, items_out, counts + base, nodes,
-                        ctx->ctl, TreeSegs{}, ctx->stream);
+      launch_leaves(plan.tile, grid[0], t4, skeys, perm, n, o4, items_out,
+                    counts, nodes, ctx->ctl, TreeSegs{}, ctx->stream);
     prev = base;
     base += grid[L];
   }
@@ -883,18 +883,17 @@ void enqueue_batch(lbvh_ctx *ctx, const float *tri, bool have_bounds,
                       T + P.o_seg_off, T + P.o_lprev0[L], T + P.o_lprev_n[L]};
     const int4 *items_in = items + kItemInt4 * kTreeFrontier * prev;
     int4 *items_out = items + kItemInt4 * kTreeFrontier * base;
-    if (P.forest)
-      launch_forest_level(L, P.level_tiles[L], t4, out, vout, P.total,
-                          reinterpret_cast<float4 *>(tri_out), items_in,
-                          counts + prev, 0u, items_out, counts + base,
-                          static_cast<float4 *>(bvh_out), ctx->ctl, ts,
-                          ctx->stream);
+    float4 *o4 = reinterpret_cast<float4 *>(tri_out);
+    float4 *nodes = static_cast<float4 *>(bvh_out);
+    if (L)
+      launch_items(P.level_tiles[L], P.total, items_in, counts + prev, 0u,
+                   items_out, counts + base, nodes, ctx->ctl, ts, ctx->stream);
+    else if (P.forest)
+      launch_forest_leaves(P.level_tiles[0], t4, out, vout, P.total, o4,
+                           items_out, counts, nodes, ctx->ctl, ts, ctx->stream);
     else
-      launch_tree_level(L, P.tile, P.level_tiles[L], t4, out, vout, P.total,
-                        reinterpret_cast<float4 *>(tri_out), items_in,
-                        counts + prev, 0u, items_out, counts + base,
-                        static_cast<float4 *>(bvh_out), ctx->ctl, ts,
-                        ctx->stream);
+      launch_leaves(P.tile, P.level_tiles[0], t4, out, vout, P.total, o4,
+                    items_out, counts, nodes, ctx->ctl, ts, ctx->stream);
     prev = base;
     base += P.level_tiles[L];
   }

@@ -237,31 +237,35 @@ struct TreeSegs {
 // Tiles of each level of an n-leaf build (returns the number of levels).
 int tree_levels(uint32_t n, int tile, uint32_t *grid);
 uint64_t tree_tiles_total(uint32_t n, int tile);
-// One agglomeration level (batched builds pass their segments).  items_in /
-// count_in: the level below's slots and counts, indexed by its tile number;
-// prev_tiles: its tile count (one mesh).
-void launch_tree_level(int level, int tile, uint32_t grid, const float4 *tri,
-                       const uint32_t *skeys, const int32_t *perm, uint32_t n,
-                       float4 *otri, const int4 *items_in,
-                       const uint32_t *count_in, uint32_t prev_tiles,
-                       int4 *items_out, uint32_t *count_out, float4 *nodes,
-                       Ctl *ctl, const TreeSegs &segs, hipStream_t s);
+// Level 0 by climbs (k_leaves), over leaf tiles of `tile` (batched builds pass
+// their segments).
+void launch_leaves(int tile, uint32_t grid, const float4 *tri,
+                   const uint32_t *skeys, const int32_t *perm, uint32_t n,
+                   float4 *otri, int4 *items_out, uint32_t *count_out,
+                   float4 *nodes, Ctl *ctl, const TreeSegs &segs,
+                   hipStream_t s);
 
 // k_forest.hip
-// One agglomeration level of at most kForestMax leaves in all, over leaf
-// tiles of kForestTile: the arguments, items and level plan of
-// launch_tree_level.  Refits, this against the best leaf tile of k_leaves:
-// 1,500 leaves 9.4 / 17.3 us, 2^16 16.3 / 24.5, 2^18 24.7 / 37, 2^20 63 / 72
-// (uniform) and 48 / 59 (heightfield), 8M 368 / 380 and 287 / 293; at 2^24 it
-// turns (838 / 798, 577 / 555).
+// Level 0 of at most kForestMax leaves in all, without climbs, over leaf tiles of
+// kForestTile.  Refits in us, this / k_leaves' tile of 1,024 under the same item
+// levels: 20,000 leaves 15.9 / 17.5, 2^16 16.4 / 21.9, 2^18 24.8 / 26.2, 500,000 40.4
+// / 36.1 (the last of two rounds of tiles is short), 1M 61.2 / 58.7, 3M 145 / 144;
+// heightfields 15.5 / 18.2, 16.7 / 23.3, 23.0 / 24.1, 33.9 / 31.1, 46.5 / 51.7, 98.5 /
+// 107, which turn at 3.6M (3.9M 158 / 140).
 constexpr int kForestTile = 256;
-constexpr uint32_t kForestMax = 1u << 23;
-void launch_forest_level(int level, uint32_t grid, const float4 *tri,
-                         const uint32_t *skeys, const int32_t *perm,
-                         uint32_t n, float4 *otri, const int4 *items_in,
-                         const uint32_t *count_in, uint32_t prev_tiles,
-                         int4 *items_out, uint32_t *count_out, float4 *nodes,
-                         Ctl *ctl, const TreeSegs &segs, hipStream_t s);
+constexpr uint32_t kForestMax = 7u << 19;
+void launch_forest_leaves(uint32_t grid, const float4 *tri,
+                          const uint32_t *skeys, const int32_t *perm,
+                          uint32_t n, float4 *otri, int4 *items_out,
+                          uint32_t *count_out, float4 *nodes, Ctl *ctl,
+                          const TreeSegs &segs, hipStream_t s);
+// An item level, over either leaf level.  items_in / count_in: the level below's
+// slots and counts, indexed by its tile number; prev_tiles: its tile count (one
+// mesh).
+void launch_items(uint32_t grid, uint32_t n, const int4 *items_in,
+                  const uint32_t *count_in, uint32_t prev_tiles,
+                  int4 *items_out, uint32_t *count_out, float4 *nodes, Ctl *ctl,
+                  const TreeSegs &segs, hipStream_t s);
 
 // k_batch.hip
 // The blocks of a batch's bounds: each block's mesh, and each mesh's first block

@@ -63,7 +63,7 @@ __device__ __forceinline__ void write_single_leaf_node(int4 *nodes, const float 
 
 constexpr int kFrontierMax = kTreeFrontier;
 // Level L-1 tiles per tile: kFanIn (up to 32 x 128 items, typically a few
-// hundred; a round holds at least kItemTile - kFrontierMax new items), or
+// hundred; a round holds at least kForestItems - kFrontierMax new ones), or
 // all of them, up to kFanInMax, in one last tile.  Depends only on the
 // number of level L-1 tiles, so the host's level plan and the kernel agree.
 constexpr int kFanIn = 32;
