@@ -32,20 +32,19 @@ __device__ __forceinline__ V3 v3(int4 v) {
   return {__int_as_float(v.x), __int_as_float(v.y), __int_as_float(v.z)};
 }
 
-// The distance of tri_intersect (pathtracer.js:587-619), -1 for a miss.
+// The distance of tri_intersect (pathtracer.js:587-619), -1 for a miss; its early
+// ends in one test.
 __device__ __forceinline__ float tri_distance(V3 o, V3 d, V3 v0, V3 v1, V3 v2) {
   const V3 e1 = sub(v1, v0), e2 = sub(v2, v0);
   const V3 pvec = cross(d, e2);
   const float det = dot(e1, pvec);
-  if (fabsf(det) < 1e-10f) return -1.f;
   const float idet = __fdiv_rn(1.0f, det);
   const V3 tvec = sub(o, v0);
   const float u = __fmul_rn(dot(tvec, pvec), idet);
-  if (u < 0.f || u > 1.f) return -1.f;
   const V3 qvec = cross(tvec, e1);
   const float v = __fmul_rn(dot(d, qvec), idet);
-  if (v < 0.f || __fadd_rn(u, v) > 1.f) return -1.f;
-  return __fmul_rn(dot(e2, qvec), idet);
+  const bool out = u < 0.f || u > 1.f || fabsf(det) < 1e-10f || v < 0.f || __fadd_rn(u, v) > 1.f;
+  return out ? -1.f : __fmul_rn(dot(e2, qvec), idet);
 }
 
 // Its normal, taken once per ray for the closest hit.
@@ -57,17 +56,20 @@ __device__ __forceinline__ V3 tri_normal(V3 v0, V3 v1, V3 v2) {
   return {__fdiv_rn(nrm.x, len), __fdiv_rn(nrm.y, len), __fdiv_rn(nrm.z, len)};
 }
 
-// aabb_intersect (pathtracer.js:621-628): entry distance or -1e30.
-__device__ __forceinline__ float aabb_intersect(V3 lo, V3 hi, V3 o, V3 inv) {
+// aabb_intersect (pathtracer.js:621-628): the entry distance t0, and whether
+// the traversal takes the child (a -1e30 there is a miss).
+__device__ __forceinline__ bool aabb_hit(V3 lo, V3 hi, V3 o, V3 inv, float dist,
+                                         float &t0) {
   const float fx = __fmul_rn(__fsub_rn(hi.x, o.x), inv.x);
   const float fy = __fmul_rn(__fsub_rn(hi.y, o.y), inv.y);
   const float fz = __fmul_rn(__fsub_rn(hi.z, o.z), inv.z);
   const float nx = __fmul_rn(__fsub_rn(lo.x, o.x), inv.x);
   const float ny = __fmul_rn(__fsub_rn(lo.y, o.y), inv.y);
   const float nz = __fmul_rn(__fsub_rn(lo.z, o.z), inv.z);
-  const float t0 = fmaxf(fminf(fx, nx), fmaxf(fminf(fy, ny), fminf(fz, nz)));
+  t0 = fmaxf(fminf(fx, nx), fmaxf(fminf(fy, ny), fminf(fz, nz)));
   const float t1 = fminf(fmaxf(fx, nx), fminf(fmaxf(fy, ny), fmaxf(fz, nz)));
-  return (t1 >= t0) ? ((t1 < 0.f) ? -1e30f : t0) : -1e30f;
+  // (t0 is NaN only where t1 is)
+  return t1 >= fmaxf(t0, 0.f) && t0 < dist && t0 != -1e30f;
 }
 
 constexpr int kRayStack = 64;  // the path tracer's is 32 (pathtracer.js:493)
@@ -88,17 +90,27 @@ constexpr uint32_t kRayChunk = 64;  // consecutive blocks on one XCD
 //   * kRayChunk blocks (4,096 rays) in a row run on one XCD, whose L2 then
 //     holds the nodes they share (1M rays of a frame over 1M triangles 398 ->
 //     317 us).
-//   * the stack's top is at hand when a step ends in a pop.
+//   * the stack's top is at hand when a step ends in a pop;
+//   * a step is straight-line code: a branch costs a wave some 16 cycles and a
+//     mask, so addresses are selected, the far child is stored above the top
+//     whether it is pushed or not, the triangle test has no early ends, and
+//     one branch holds all of the stack past LDS.
 // Together 245 -> 172 us for a 512 x 512 frame over 100,000 clustered
-// triangles (186 before the last), 1,000 -> 740 us for 1M scattered rays over 1M.  Dropping popped
-// nodes beyond the closest hit lost (the stack entries double), and so did
-// descending to a leaf per lane before any test, and touching both children
-// ahead.
+// triangles (186 before the last but one), 1,000 -> 740 us for 1M scattered rays over 1M;
+// the last by wall clock: that frame 222 -> 197, a 1,024 x 1,024 frame over a
+// heightfield of 500,000 250 -> 221, 2^14 scattered rays over 4,097 triangles 65
+// -> 54, 1M over 1M uniform 1,150 -> 1,131, 1M over a surface of 300,000 540 ->
+// 547.  Dropping popped nodes beyond the closest hit lost (the stack entries
+// double), and so did descending to a leaf per lane before any test, touching
+// both children ahead, a step that takes a leaf together with the node that
+// comes off the stack after it (the frame 244), and a higher priority for waves
+// with many steps (235).
 __global__ __launch_bounds__(kRayThreads) void k_raycast(
     const int4 *__restrict__ nodes, const int4 *__restrict__ tri, uint32_t n,
     const float4 *__restrict__ rays, uint32_t count, float4 *__restrict__ hits,
     uint32_t max_steps) {
-  __shared__ int s_stack[kRayLds][kRayThreads];
+  // entry k in row k + 1; row 0: of an empty stack; the last one: past them
+  __shared__ int s_stack[kRayLds + 2][kRayThreads];
   int deep[kRayStack - kRayLds];
   const uint32_t tid = threadIdx.x;
   // chunks of kRayChunk blocks go to the XCDs in turn; the rest as they come
@@ -123,43 +135,44 @@ __global__ __launch_bounds__(kRayThreads) void k_raycast(
   int node = 0;
   for (uint32_t step = 0; sp >= 0 && step < max_steps; ++step) {
     const bool leaf = node < 0;
-    const uint32_t id = leaf ? (uint32_t)(-(node + 1)) : (uint32_t)node;
-    if (!leaf && id >= n) break;
-    const int4 *at = leaf ? tri + 3 * (size_t)(id < n ? id : 0u)
-                          : nodes + 4 * (size_t)id;
-    const int4 a = at[0], b = at[1], c = at[2], e = at[leaf ? 2 : 3];
+    const uint32_t id = (uint32_t)(leaf ? ~node : node);
+    const bool in = id < n;
+    const char *base = leaf ? reinterpret_cast<const char *>(tri)
+                            : reinterpret_cast<const char *>(nodes);
+    const char *at = base + (uint64_t)(in ? id : 0u) * (leaf ? 48u : 64u);
+    const int4 *at4 = reinterpret_cast<const int4 *>(at);
+    const int4 a = at4[0], b = at4[1], c = at4[2];
+    const int4 e = *reinterpret_cast<const int4 *>(at + (leaf ? 32 : 48));
     // The stack's top, read from LDS while those loads are under way.  (Read
     // when it is popped, from LDS or scratch by its depth, it was one generic
     // load, which waits on the vector memory path.)
-    int top = s_stack[min(max(sp - 1, 0), kRayLds - 1)][tid];
-    bool next;  // the next node comes off the stack
+    const int row = min(sp, kRayLds);
+    int top = s_stack[row][tid], far = 0;
+    bool pop, push = false;
     if (leaf) {
       const float h = tri_distance(o, d, v3(a), v3(b), v3(c));
-      if (id < n && h > 0.f && h < dist) {
-        dist = h;
-        hit = id;
-      }
-      next = true;
+      const bool closer = in && h > 0.f && h < dist;
+      dist = closer ? h : dist;
+      hit = closer ? id : hit;
+      pop = true;
     } else {
-      const float ld = aabb_intersect(v3(a), v3(b), o, inv);
-      const float rdist = aabb_intersect(v3(c), v3(e), o, inv);
-      const bool lv = ld != -1e30f && ld < dist;
-      const bool rv = rdist != -1e30f && rdist < dist;
-      const bool left = lv && (!rv || ld < rdist);  // the nearer child first
-      if (lv && rv) {
-        const int far = left ? c.w : a.w;
-        if (sp < kRayLds) s_stack[sp][tid] = far;
-        else if (sp < kRayStack) deep[sp - kRayLds] = far;
-        sp = sp + 1 < kRayStack ? sp + 1 : kRayStack;
-      }
+      float lt, rt;
+      const bool lv = aabb_hit(v3(a), v3(b), o, inv, dist, lt);
+      const bool rv = aabb_hit(v3(c), v3(e), o, inv, dist, rt);
+      const bool left = lv && (!rv || lt < rt);  // the nearer child first
+      far = left ? c.w : a.w;
       node = left ? a.w : c.w;
-      next = !lv && !rv;
+      s_stack[row + 1][tid] = far;  // above the top if not pushed
+      push = in && lv && rv;
+      pop = !in || !(lv || rv);
+      sp = in ? sp : 0;
     }
-    if (next) {
-      sp -= 1;
-      if (sp >= kRayLds) top = deep[sp - kRayLds];
-      node = top;
+    if (sp >= kRayLds) {
+      if (push && sp < kRayStack) deep[sp - kRayLds] = far;
+      if (pop && sp > kRayLds) top = deep[sp - 1 - kRayLds];
     }
+    node = pop ? top : node;
+    sp = pop ? sp - 1 : min(sp + (push ? 1 : 0), kRayStack);
   }
   // RayHit: normal facing the ray, dist -1 for a miss (pathtracer.js:572-583)
   V3 nrm = {0.f, 0.f, 0.f};
