@@ -344,22 +344,35 @@ __global__ __launch_bounds__(kForestLeaves) void k_forest_leaves(
   static_assert(3 * 64 <= kTable, "a wave's triangles");
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   int4 *stage = reinterpret_cast<int4 *>(&L.a[w][0]);
-  if (tid < m) {
-    const uint32_t pi = (uint32_t)perm[k];
-    const uint32_t k_here = skeys[k];
-    const uint32_t k_next = skeys[k + 1 < N ? k + 1 : k];
+  {
+    const uint32_t kc = min(k, N - 1);  // a lane past the mesh: the last leaf
+    const uint32_t pi = (uint32_t)perm[kc];
+    const uint32_t k_here = skeys[kc];
+    const uint32_t k_next = skeys[min(k + 1, N - 1)];
     const uint32_t k_0 = skeys[ts], k_prev = skeys[ts > 0 ? ts - 1 : 0];
-    const size_t src = 3 * (size_t)(pi < N ? pi : 0u);
-    const int4 a = tri[src], b = tri[src + 1], c = tri[src + 2];
-    stage[3 * lane] = a;
-    stage[3 * lane + 1] = b;
-    stage[3 * lane + 2] = c;
-    tri_box(a, b, c, mn, mx);
-    perturb(mn, mx);
+    int4 a, b, c;
+    if (scattered_gather(pi)) {
+      gather_rows(tri, pi, N, stage);
+      a = stage[3 * lane];
+      b = stage[3 * lane + 1];
+      c = stage[3 * lane + 2];
+    } else if (tid < m) {
+      const size_t src = 3 * (size_t)(pi < N ? pi : 0u);
+      a = tri[src];
+      b = tri[src + 1];
+      c = tri[src + 2];
+      stage[3 * lane] = a;
+      stage[3 * lane + 1] = b;
+      stage[3 * lane + 2] = c;
+    }
     const int d_next = delta_next(k_here, k_next, k);
     const int d_prev = delta_next(k_prev, k_0, (uint32_t)(ts - 1));
-    d = k + 1 < N ? d_next : -1;
-    d0 = ts > 0 ? d_prev : -1;
+    if (tid < m) {
+      tri_box(a, b, c, mn, mx);
+      perturb(mn, mx);
+      d = k + 1 < N ? d_next : -1;
+      d0 = ts > 0 ? d_prev : -1;
+    }
   }
   wave_lds_fence();
   {

@@ -1023,7 +1023,7 @@ __device__ __forceinline__ void climb_leaves(Climb &c, LeafLds<T> &L, int n,
 // boxes, climbs, writes the tile's nodes and its frontier.  With segments
 // (batched builds) every segment is an independent mesh: positions, node ids
 // and the permutation are relative to its first leaf.
-template <int T>
+template <int T, bool kSegs>
 __global__ __launch_bounds__(T) void k_leaves(
     const int4 *__restrict__ tri_all, const uint32_t *__restrict__ skeys_all,
     const int32_t *__restrict__ perm_all, uint32_t n_all,
@@ -1034,7 +1034,7 @@ __global__ __launch_bounds__(T) void k_leaves(
   const int tid = threadIdx.x;
   const uint32_t gtile = xcd_tile(blockIdx.x, gridDim.x);
   uint32_t tile0 = 0, leaf_base = 0, N = n_all;
-  if (segs.tile_seg) {
+  if (kSegs) {
     const uint32_t sg = segs.tile_seg[gtile];
     tile0 = segs.seg_tile0[sg];
     leaf_base = segs.seg_off[sg];
@@ -1054,34 +1054,50 @@ __global__ __launch_bounds__(T) void k_leaves(
   c.l = c.r = k;
   L.cnt[tid] = 0u;
   L.gap_of[tid] = -1;
-  if (active) {
+  {
     // Every load that does not depend on the permutation goes out with it
     // (the keys at the leaf's gaps, clamped to the mesh so no branch
     // separates them): the tile waits two round trips, the permutation and
     // then the gather it names, instead of three.
-    const uint32_t pi = (uint32_t)perm_all[leaf_base + k];
-    const uint32_t k_here = skeys[k];
-    const uint32_t k_next = skeys[(uint32_t)k + 1 < N ? k + 1 : k];
-    const uint32_t k_prev = skeys[k > 0 ? k - 1 : k];  // thread 0's gap
-    const size_t src = 3 * (size_t)(leaf_base + (pi < N ? pi : 0u));
-    // plain loads: neighbouring leaves gather triangles that share lines, and
-    // the L2 keeps them (non-temporal loads took the level 0.53 -> 0.65 ms)
-    const int4 a = tri_all[src], b = tri_all[src + 1], d = tri_all[src + 2];
+    const uint32_t kc = min((uint32_t)k, N - 1);  // a lane past the mesh: the last leaf
+    const uint32_t pi = (uint32_t)perm_all[leaf_base + kc];
+    const uint32_t k_here = skeys[kc];
+    const uint32_t k_next = skeys[min((uint32_t)k + 1, N - 1)];
+    const uint32_t k_prev = skeys[kc > 0 ? kc - 1 : kc];  // thread 0's gap
     // O_TRI goes out through LDS (the node slots are free until the climb):
     // a lane's own 48-byte row would put 48 bytes between the lanes of each
-    // store, where the staged rows are stored 16 contiguous bytes per lane
-    int4 *stage = &L.node[0][0];
-    stage[3 * tid] = a;
-    stage[3 * tid + 1] = b;
-    stage[3 * tid + 2] = d;
-    tri_box(a, b, d, c.mn, c.mx);
-    perturb(c.mn, c.mx);
+    // store, where the staged rows are stored 16 contiguous bytes per lane.
+    // The gather takes plain loads: neighbouring leaves gather triangles that
+    // share lines, and the L2 keeps them (non-temporal loads took the level
+    // 0.53 -> 0.65 ms).
+    const int lane = tid & 63, w0 = tid - lane;
+    int4 *stage = &L.node[0][0] + 3 * w0;  // the wave's
+    int4 a, b, d;
+    const bool scattered = scattered_gather(pi);
+    if (scattered) {
+      gather_rows(tri_all + 3 * (size_t)leaf_base, pi, N, stage);
+      a = stage[3 * lane];
+      b = stage[3 * lane + 1];
+      d = stage[3 * lane + 2];
+    } else if (active) {
+      const size_t src = 3 * (size_t)(leaf_base + (pi < N ? pi : 0u));
+      a = tri_all[src];
+      b = tri_all[src + 1];
+      d = tri_all[src + 2];
+      stage[3 * lane] = a;
+      stage[3 * lane + 1] = b;
+      stage[3 * lane + 2] = d;
+    }
     // both deltas computed unconditionally and selected, so the compiler
     // does not sink their loads into branches behind the gather
     const int d_next = delta_next(k_here, k_next, (uint32_t)k);
     const int d_prev = delta_next(k_prev, k_here, (uint32_t)(k - 1));
-    L.dgap[tid + 1] = ((uint32_t)k + 1 < N) ? d_next : -1;
-    if (tid == 0) L.dgap[0] = k > 0 ? d_prev : -1;
+    if (active) {
+      tri_box(a, b, d, c.mn, c.mx);
+      perturb(c.mn, c.mx);
+      L.dgap[tid + 1] = ((uint32_t)k + 1 < N) ? d_next : -1;
+      if (tid == 0) L.dgap[0] = k > 0 ? d_prev : -1;
+    }
   }
   __syncthreads();
   {
@@ -1265,7 +1281,8 @@ static void launch_leaf_level(uint32_t grid, const int4 *t4,
                               uint32_t n, int4 *o4, int4 *items_out,
                               uint32_t *count_out, int4 *n4, Ctl *ctl,
                               const TreeSegs &segs, hipStream_t s) {
-  hipLaunchKernelGGL(k_leaves<T>, dim3(grid), dim3(T), 0, s, t4, skeys, perm,
+  hipLaunchKernelGGL((segs.tile_seg ? k_leaves<T, true> : k_leaves<T, false>),
+                     dim3(grid), dim3(T), 0, s, t4, skeys, perm,
                      n, o4, items_out, count_out, n4, ctl, segs);
 }
 

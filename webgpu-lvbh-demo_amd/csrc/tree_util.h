@@ -61,6 +61,42 @@ __device__ __forceinline__ void write_single_leaf_node(int4 *nodes, const float 
   nodes[3] = make_int4(0, 0, 0, 0);
 }
 
+// The gather of a wave's triangles through the permutation has two forms: a
+// lane loads its own 48-byte row in three instructions, each of them touching a
+// line per lane, or three lanes load a row, 16 contiguous bytes each, and an
+// instruction touches a third as many.  Where the leaves' triangles are scattered
+// and still in a cache (batched meshes, up to 5M triangles) the lines an
+// instruction touches set the gather's time and the second form is faster: 80M
+// triangles in 2,048 random meshes 5,710 -> 5,480 us, 5M random ones 420 -> 409.
+// Where neighbouring leaves share lines the first is (16M heightfield 1,052,
+// 1,062 with the second; batches of 80M surface triangles 5,080 / 5,160), so a wave
+// picks by its own leaves: scattered if of its pairs of neighbours fewer than a
+// quarter come from nearby triangles.  The two branches cost a 1M heightfield
+// 139.0 -> 139.7 us.  Every lane of the wave calls it.
+__device__ __forceinline__ bool scattered_gather(uint32_t pi) {
+  const uint32_t other = (uint32_t)__shfl_xor((int)pi, 1, 64);
+  return __popcll(__ballot(max(pi, other) - min(pi, other) < 16u)) < 16;
+}
+
+// Triangles of the wave's leaves into stage (192 int4s of LDS) with 16
+// contiguous bytes per lane, three lanes per triangle.  Every lane of the wave
+// calls it, with a leaf's triangle.
+__device__ __forceinline__ void gather_rows(const int4 *tri, uint32_t pi,
+                                            uint32_t N, int4 *stage) {
+  const int lane = threadIdx.x & 63;
+  int4 v[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const int e = j * 64 + lane;
+    const uint32_t p = (uint32_t)__shfl((int)pi, e / 3, 64);
+    v[j] = tri[3 * (size_t)(p < N ? p : 0u) + e % 3];
+  }
+#pragma unroll
+  for (int j = 0; j < 3; ++j) stage[j * 64 + lane] = v[j];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 constexpr int kFrontierMax = kTreeFrontier;
 // Level L-1 tiles per tile: kFanIn (up to 32 x 128 items, typically a few
 // hundred; a round holds at least kForestItems - kFrontierMax new ones), or
