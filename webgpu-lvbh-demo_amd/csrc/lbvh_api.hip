@@ -66,6 +66,7 @@ struct lbvh_ctx {
   DevBuf b_keys_a, b_keys_b, b_idx_a, b_idx_b, b_digits, b_bounds,
       b_tree_items, b_tree_counts, b_table, b_cen;
   struct BatchPlan {
+    bool ready = false;  // its tables are in b_table
     std::vector<uint32_t> offsets;
     int tile = 0, bits = kRadixBits, items = kSortItems;
     bool forest = false;
@@ -762,8 +763,8 @@ int make_plan(lbvh_ctx *ctx, const uint32_t *offsets, uint32_t S) {
   TreePlan plan = tree_plan(ctx, offsets[S]);
   if (!plan.forest) plan.tile = tile_for(ctx, big);
   const int items = batch_sort_items(ctx, offsets[S]);
-  if (P.S == S && P.items == items && P.tile == plan.tile && P.forest == plan.forest &&
-      P.bits == bits_for(ctx, offsets[S]) &&
+  if (P.ready && P.S == S && P.items == items && P.tile == plan.tile &&
+      P.forest == plan.forest && P.bits == bits_for(ctx, offsets[S]) &&
       std::equal(P.offsets.begin(), P.offsets.end(), offsets) &&
       P.offsets.size() == (size_t)S + 1)
     return LBVH_OK;
@@ -834,6 +835,7 @@ int make_plan(lbvh_ctx *ctx, const uint32_t *offsets, uint32_t S) {
   HIP_TRY(ctx, hipMemcpyAsync(ctx->b_table.ptr, tab.data(), 4ull * tab.size(),
                               hipMemcpyHostToDevice, ctx->stream));
   HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+  P.ready = true;
   return LBVH_OK;
 }
 
