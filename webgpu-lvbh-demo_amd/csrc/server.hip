@@ -32,6 +32,7 @@
 #include "../../include/lbvh.h"
 #include "lbvh_internal.h"
 #include "range_arena.h"
+#include "result_ring.h"
 #include "synth_math.h"
 
 namespace lbvh {
@@ -228,7 +229,7 @@ struct Slot {
   // twice.
   uint64_t max_build_n = 0, max_refit_n = 0;
   uint64_t bound = 0;
-  uint32_t next_serial = 1;  // dispatcher only; results entry serial % depth
+  lbvh::ResultRing<kSlotDepth> ring;  // dispatcher only
   // kSlotDepth entries: what a request's epilogue left (pinned host memory,
   // and its device address), and the device words its digest accumulates in
   RequestResult *results = nullptr;
@@ -684,11 +685,10 @@ void dispatcher(lbvh_server *s) {
         w.req = std::move(*qi);
         qi = s->queue.erase(qi);
         w.start_s = now_s();
-        w.serial = sl.next_serial++;
-        w.ring = (int)(w.serial % kSlotDepth);
         w.digest = s->digest;
-        st = prepare(s, w);
+        st = sl.ring.admit(&w.serial, [&] { return prepare(s, w); });
         if (st == LBVH_OK) {
+          w.ring = sl.ring.entry(w.serial);
           {
             std::lock_guard<std::mutex> g(sl.m);
             sl.mailbox.push_back(std::move(w));
