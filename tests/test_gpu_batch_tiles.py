@@ -1,0 +1,36 @@
+"""The sort tiles of a batch by its largest mesh: 1,024 keys up to 65,536 keys
+(32,768 of more than 2^20 in all; 16,384 and 4,096 with 10-bit digits), 4,096 beyond, where one block's scan of a mesh's
+small tiles would be the longer chain.  The tiles show in the scratch that the
+context holds, beside one under a budget, which always takes the large ones."""
+import numpy as np
+import pytest
+
+from test_gpu_batched import make_batch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("past", [False, True], ids=["at the line", "past it"])
+@pytest.mark.parametrize("bits,most,rest", [
+    (8, 65536, []), (8, 65536, [2000] * 40), (8, 65536, [7, 0, 1025] * 100), (8, 32768, [3000] * 400),
+    (10, 16384, []), (10, 16384, [2000] * 40), (10, 16384, [7, 0, 1025] * 100), (10, 4096, [3000] * 400)])
+def test_tiles_follow_the_largest_mesh(lb, ora, bits, most, rest, past):
+    meshes, offsets, tri = make_batch(lb, rest[:3] + [most + past] + rest[3:], 70)
+    total = int(offsets[-1])
+    held, outs = [], []
+    for budget in (0, 8 << 30):
+        with lb.Context(0, hbm_budget=budget) as c:
+            c.set_tuning(lb.TUNE_SORT_BITS, bits)
+            c.set_tuning(lb.TUNE_TREE_TILE, 1024)  # the same tree either way
+            d, bvh, otri = c.to_device(tri), c.alloc(64 * total), c.alloc(48 * total)
+            c.build_batched(d, offsets, None, bvh, otri)
+            outs.append((bvh.read(np.uint8, 64 * total), otri.read(np.uint32, 12 * total)))
+            held.append(c.bytes_in_use())
+    assert (held[0] == held[1]) == past, held
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
+    for k in (0, min(3, len(meshes) - 1), len(meshes) - 1):
+        a, b = int(offsets[k]), int(offsets[k + 1])
+        wb, wo = ora.build(meshes[k], None, 0)[:2]
+        assert np.array_equal(outs[0][0][64 * a:64 * b], wb), k
+        assert np.array_equal(outs[0][1][12 * a:12 * b], wo.view(np.uint32).ravel()), k

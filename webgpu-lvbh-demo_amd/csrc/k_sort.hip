@@ -10,7 +10,7 @@
 // words per tile).
 //
 // Each pass is reduce-then-scan over tiles of kSortTile keys (kSmallSortTile
-// for a single mesh of at most kSmallSortMax keys, a batch of at most
+// for a single mesh of at most kSmallSortMax keys, a batch of small meshes,
 // kBatchSmallMax):
 //   count    per-tile digit counts (pass 0's are written by the Morton
 //            kernel as it produces the keys), and their column sums;

@@ -479,10 +479,12 @@ TreePlan tree_plan(const lbvh_ctx *ctx, uint32_t n) {
   return {tile, false};
 }
 
-// Keys per thread of a batched sort of n keys in all: the small tile as for a
-// single mesh, but not under an HBM budget (four times the tiles' counts).
-int batch_sort_items(const lbvh_ctx *ctx, uint32_t n) {
-  return ctx->budget == 0 && n <= kBatchSmallMax ? kSmallSortItems : kSortItems;
+// Keys per thread of a batched sort of n keys in all, at most `big` a mesh: the
+// small tile as for a single mesh where the meshes are small, but not under an HBM
+// budget (four times the tiles' counts).
+int batch_sort_items(const lbvh_ctx *ctx, uint32_t n, uint32_t big, int bits) {
+  const bool small = n <= kBatchSmallMax && big <= batch_small_mesh(n, bits);
+  return ctx->budget == 0 && small ? kSmallSortItems : kSortItems;
 }
 
 int bits_for(const lbvh_ctx *ctx, uint32_t n) {
@@ -762,9 +764,12 @@ int make_plan(lbvh_ctx *ctx, const uint32_t *offsets, uint32_t S) {
   // the trees' levels run together: k_forest.hip's up to as many leaves in all
   TreePlan plan = tree_plan(ctx, offsets[S]);
   if (!plan.forest) plan.tile = tile_for(ctx, big);
-  const int items = batch_sort_items(ctx, offsets[S]);
+  // one segmented sort runs over all the keys: its digit width is that of
+  // a sort of the total
+  const int bits = bits_for(ctx, offsets[S]);
+  const int items = batch_sort_items(ctx, offsets[S], big, bits);
   if (P.ready && P.S == S && P.items == items && P.tile == plan.tile &&
-      P.forest == plan.forest && P.bits == bits_for(ctx, offsets[S]) &&
+      P.forest == plan.forest && P.bits == bits &&
       std::equal(P.offsets.begin(), P.offsets.end(), offsets) &&
       P.offsets.size() == (size_t)S + 1)
     return LBVH_OK;
@@ -774,9 +779,7 @@ int make_plan(lbvh_ctx *ctx, const uint32_t *offsets, uint32_t S) {
   P.tile = plan.tile;
   P.forest = plan.forest;
   P.items = items;
-  // one segmented sort runs over all the keys: its digit width is that of
-  // a sort of the total
-  P.bits = bits_for(ctx, offsets[S]);
+  P.bits = bits;
   P.total = offsets[S];
   std::vector<uint32_t> tab;
   auto put = [&](const std::vector<uint32_t> &v) {

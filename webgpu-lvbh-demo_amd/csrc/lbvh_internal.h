@@ -45,7 +45,20 @@ constexpr uint32_t kSmallSortMax = 1u << 20;
 // Batched sorts of at most this many keys in all use the small tile too: 17,555
 // keys in 16 meshes 81.6 / 61.9 us a batch, 713,000 in 300 141 / 107, 4.8M in
 // 700 450 / 429 (4,096 / 1,024 keys); 18M in 1,000 turns, 1,438 / 1,535.
+// But one block scans a mesh's tile counts, so a large mesh's small tiles are a
+// long chain, with 10-bit digits, whose tiles hold four times the counts, the
+// longer: the meshes must have at most so many keys each (batch_small_mesh).
+// Batches in us, 4,096 / 1,024 keys.  8 bits, up to kSmallSortMax in all: 65,536 with
+// 200 meshes of 2,000 125 / 122, 131,072 with those 144 / 164 (a few meshes turn
+// later: 4 of 131,072 132 / 124, of 200,000 160 / 158); more: 100 of 32,768 290 / 285,
+// 60 of 65,536 329 / 340, 5M alone 634 / 1,226.  10 bits: 16,384 alone 84 / 76, 4 of
+// 32,768 98 / 108, 100,003 alone 128 / 187; more: 280 of 4,096 144 / 133, 500 of 4,096
+// 187 / 190, 240 of 8,192 187 / 201, 1M with 500 of 2,000 530 / 1,433.
 constexpr uint32_t kBatchSmallMax = 1u << 23;
+inline uint32_t batch_small_mesh(uint32_t n, int bits) {
+  if (bits == kWideBits) return n <= kSmallSortMax ? 1u << 14 : 1u << 12;
+  return n <= kSmallSortMax ? 1u << 16 : 1u << 15;
+}
 
 constexpr int kTreeTileDefault = 1024;  // leaves per tile of the fused up pass
 constexpr int kMaxTreeLevels = 16;      // agglomeration levels (6 at 2^24, T=1024)
