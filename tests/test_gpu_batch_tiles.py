@@ -1,6 +1,7 @@
-"""The sort tiles of a batch by its largest mesh: 1,024 keys up to 65,536 keys
-(32,768 of more than 2^20 in all; 16,384 and 4,096 with 10-bit digits), 4,096 beyond, where one block's scan of a mesh's
-small tiles would be the longer chain.  The tiles show in the scratch that the
+"""The sort tiles of a batch by its largest mesh: 1,024 keys up to the line that its
+size in all, its digits and its number of meshes give (batch_small_mesh of
+csrc/lbvh_internal.h), 4,096 beyond, where one block's scan of a mesh's small tiles
+would be the longer chain.  The tiles show in the scratch that the
 context holds, beside one under a budget, which always takes the large ones."""
 import numpy as np
 import pytest
@@ -12,8 +13,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("past", [False, True], ids=["at the line", "past it"])
 @pytest.mark.parametrize("bits,most,rest", [
-    (8, 65536, []), (8, 65536, [2000] * 40), (8, 65536, [7, 0, 1025] * 100), (8, 32768, [3000] * 400),
-    (10, 16384, []), (10, 16384, [2000] * 40), (10, 16384, [7, 0, 1025] * 100), (10, 4096, [3000] * 400)])
+    (8, 3 << 16, []), (8, 3 << 16, [2000] * 40), (8, 65536, [7, 0, 1025] * 100), (8, 65536, [2000] * 200),
+    (8, 32768, [3000] * 400), (10, 5 << 12, []), (10, 5 << 12, [20000] * 4), (10, 16384, [7, 0, 1025] * 100),
+    (10, 4096, [3000] * 400)])
 def test_tiles_follow_the_largest_mesh(lb, ora, bits, most, rest, past):
     meshes, offsets, tri = make_batch(lb, rest[:3] + [most + past] + rest[3:], 70)
     total = int(offsets[-1])

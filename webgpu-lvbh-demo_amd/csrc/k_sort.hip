@@ -246,10 +246,7 @@ __global__ __launch_bounds__(kThreads) void k_scan_columns(
 // tiles each, thread t of a group its digits [t * kDpt, (t + 1) * kDpt), tile
 // after tile (each tile's R words in one coalesced sweep of the group), kUnroll
 // tiles in flight; the groups' sums and a scan over the digits give each its
-// first positions.  An empty segment has no tiles.  One group takes 9 us for a
-// mesh of 64 tiles, the chain of its loads, four 5; but four where blocks fill
-// the chip cost more (300 meshes 4.8 against 3.6 us, 1,000 8.8 against 6.2).
-constexpr uint32_t kFewSegs = 256;  // at most so many segments: four groups
+// first positions.  An empty segment has no tiles.
 template <int kBits, int kSegGroups>
 __global__ __launch_bounds__(kSegGroups *kSortThreads) void k_seg_scan(
     const uint32_t *__restrict__ cnt, uint32_t *__restrict__ off,
@@ -643,7 +640,7 @@ void sort_pass(int pass, const uint32_t *keys_in, const int32_t *vals_in,
   const int small = !segmented && tiles <= kSmallScanTiles;
   const uint32_t *offs = small ? cnt : off;
   if (segmented) {
-    if (num_segs <= kFewSegs && tiles > 4 * num_segs)
+    if (seg_scan_groups(num_segs, tiles) == 4)
       hipLaunchKernelGGL((k_seg_scan<kBits, 4>), dim3(num_segs),
                          dim3(4 * kSortThreads), 0, s, cnt, off, tiles, sg,
                          num_segs);

@@ -479,12 +479,22 @@ TreePlan tree_plan(const lbvh_ctx *ctx, uint32_t n) {
   return {tile, false};
 }
 
-// Keys per thread of a batched sort of n keys in all, at most `big` a mesh: the
-// small tile as for a single mesh where the meshes are small, but not under an HBM
-// budget (four times the tiles' counts).
-int batch_sort_items(const lbvh_ctx *ctx, uint32_t n, uint32_t big, int bits) {
-  const bool small = n <= kBatchSmallMax && big <= batch_small_mesh(n, bits);
-  return ctx->budget == 0 && small ? kSmallSortItems : kSortItems;
+// Keys per thread of a batched sort: the small tile as for a single mesh where the
+// meshes are small (batch_small_mesh), but not under an HBM budget (four times the
+// tiles' counts).
+int batch_sort_items(const lbvh_ctx *ctx, const uint32_t *offsets, uint32_t S,
+                     int bits) {
+  const uint32_t n = offsets[S];
+  if (ctx->budget || n > kBatchSmallMax) return kSortItems;
+  uint32_t big = 0, tiles = 0;
+  for (uint32_t k = 0; k < S; ++k) {
+    const uint32_t m = offsets[k + 1] - offsets[k];
+    big = std::max(big, m);
+    tiles += batch_sort_tiles(m, kSmallSortItems);
+  }
+  return big <= batch_small_mesh(n, bits, seg_scan_groups(S, tiles))
+             ? kSmallSortItems
+             : kSortItems;
 }
 
 int bits_for(const lbvh_ctx *ctx, uint32_t n) {
@@ -767,7 +777,7 @@ int make_plan(lbvh_ctx *ctx, const uint32_t *offsets, uint32_t S) {
   // one segmented sort runs over all the keys: its digit width is that of
   // a sort of the total
   const int bits = bits_for(ctx, offsets[S]);
-  const int items = batch_sort_items(ctx, offsets[S], big, bits);
+  const int items = batch_sort_items(ctx, offsets, S, bits);
   if (P.ready && P.S == S && P.items == items && P.tile == plan.tile &&
       P.forest == plan.forest && P.bits == bits &&
       std::equal(P.offsets.begin(), P.offsets.end(), offsets) &&

@@ -47,17 +47,27 @@ constexpr uint32_t kSmallSortMax = 1u << 20;
 // 700 450 / 429 (4,096 / 1,024 keys); 18M in 1,000 turns, 1,438 / 1,535.
 // But one block scans a mesh's tile counts, so a large mesh's small tiles are a
 // long chain, with 10-bit digits, whose tiles hold four times the counts, the
-// longer: the meshes must have at most so many keys each (batch_small_mesh).
-// Batches in us, 4,096 / 1,024 keys.  8 bits, up to kSmallSortMax in all: 65,536 with
-// 200 meshes of 2,000 125 / 122, 131,072 with those 144 / 164 (a few meshes turn
-// later: 4 of 131,072 132 / 124, of 200,000 160 / 158); more: 100 of 32,768 290 / 285,
-// 60 of 65,536 329 / 340, 5M alone 634 / 1,226.  10 bits: 16,384 alone 84 / 76, 4 of
-// 32,768 98 / 108, 100,003 alone 128 / 187; more: 280 of 4,096 144 / 133, 500 of 4,096
-// 187 / 190, 240 of 8,192 187 / 201, 1M with 500 of 2,000 530 / 1,433.
+// longer, and less so in four groups of threads (seg_scan_groups): the meshes must
+// have at most so many keys each.  Batches in us, 4,096 / 1,024 keys.
+//   8 bits, up to kSmallSortMax in all: 65,536 with 200 meshes of 2,000 125 / 122,
+//   131,072 with those 144 / 164; in four groups 200,000 alone 132 / 116, 5 of them 171 /
+//   170, 131,072 with 40 of 2,000 130 / 102, 4 of 262,144 163 / 181.  More in all: 100 of
+//   32,768 290 / 285, 60 of 65,536 329 / 340, 5M alone 634 / 1,226.
+//   10 bits: 16,384 with 300 of 300 89 / 83, 24,576 with those 96 / 96; in four groups
+//   20,000 alone 96 / 84, 32,768 alone 91 / 101, 100,003 alone 128 / 187.  More in all: 280
+//   of 4,096 144 / 133, 500 of 4,096 187 / 190, 240 of 8,192 187 / 201, 1M with 500 of
+//   2,000 530 / 1,433.
 constexpr uint32_t kBatchSmallMax = 1u << 23;
-inline uint32_t batch_small_mesh(uint32_t n, int bits) {
-  if (bits == kWideBits) return n <= kSmallSortMax ? 1u << 14 : 1u << 12;
-  return n <= kSmallSortMax ? 1u << 16 : 1u << 15;
+inline uint32_t batch_small_mesh(uint32_t n, int bits, int groups) {
+  if (n > kSmallSortMax) return bits == kWideBits ? 1u << 12 : 1u << 15;
+  if (groups == 1) return bits == kWideBits ? 1u << 14 : 1u << 16;
+  return bits == kWideBits ? 5u << 12 : 3u << 16;
+}
+// Groups of threads that share a mesh's scan (k_seg_scan).  One takes 9 us for a
+// mesh of 64 tiles, the chain of its loads, four 5; but four where blocks fill the
+// chip cost more (300 meshes 4.8 against 3.6 us, 1,000 8.8 against 6.2).
+inline int seg_scan_groups(uint32_t num_segs, uint32_t tiles) {
+  return num_segs <= 256 && tiles > 4 * num_segs ? 4 : 1;
 }
 
 constexpr int kTreeTileDefault = 1024;  // leaves per tile of the fused up pass
