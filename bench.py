@@ -125,6 +125,16 @@ def per_build_ms(ctx, hip, d_tri, n, bounds, bvh, otri, runs):
     return out
 
 
+def build_route(lb, ctx, n, fixed_tile=0, fixed_bits=0):
+    """Leaf tile and sort digit width that a build of n triangles takes in a
+    context without a budget (lbvh_tunable in include/lbvh.h); no width where it
+    merges sorted tiles."""
+    tile = ctx.get_tuning_for(lb.TUNE_TREE_TILE, n)
+    bits = ctx.get_tuning_for(lb.TUNE_SORT_BITS, n)
+    return {"tree_tile": tile if fixed_tile or n > 3670016 else 256,
+            "sort_digit_bits": bits if fixed_bits or n > 393216 else None}
+
+
 def small_builds_bench(lb, ctx, hip, runs=50, log=print):
     """Latency of single builds of the small configurations (uniform-64k,
     clustered-1m) on a context already tuned for their sizes: the median and
@@ -141,8 +151,7 @@ def small_builds_bench(lb, ctx, hip, runs=50, log=print):
         each = per_build_ms(ctx, hip, d, n, None, bvh, otri, runs)
         ms, _ = timed_builds(lb, ctx, hip, d, n, None, bvh, otri, runs)
         out[name] = {"triangles": n,
-                     "tree_tile": ctx.get_tuning_for(lb.TUNE_TREE_TILE, n),
-                     "sort_digit_bits": ctx.get_tuning_for(lb.TUNE_SORT_BITS, n),
+                     **build_route(lb, ctx, n),
                      "median_ms": round(each[len(each) // 2], 4),
                      "min_ms": round(each[0], 4),
                      "back_to_back_ms": round(ms / runs, 4)}
@@ -441,8 +450,7 @@ def main():
         ctx.build(d_tri, n, None, bvh, otri)
     ctx.synchronize()
 
-    tile = ctx.get_tuning_for(lb.TUNE_TREE_TILE, n)
-    bits = ctx.get_tuning_for(lb.TUNE_SORT_BITS, n)
+    route = build_route(lb, ctx, n, args.tree_tile, args.sort_bits)
     log(f"timed x{args.steps}")
     ms, wall = timed_builds(lb, ctx, hip, d_tri, n, None, bvh, otri, args.steps)
     ms_per_step = ms / args.steps
@@ -576,7 +584,7 @@ def main():
         "dtype": "fp32+u32",
         "data": "synthetic",
         "config": {"workload": args.workload, "triangles": n,
-                   "tree_tile": tile, "sort_digit_bits": bits,
+                   **route,
                    "bounds": "GPU reduction", "div_mode": "mul_rcp",
                    "inputs": "resident in HBM"},
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": round(dom_gbs, 1),

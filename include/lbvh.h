@@ -95,30 +95,32 @@ int lbvh_get_div_mode(const lbvh_ctx *ctx);
  * are validated; results do not depend on them. */
 typedef enum {
   LBVH_TUNE_TREE_TILE = 0, /* leaves per block of the fused up pass:
-                              256|512|1024.  Not fixed, builds and refits of
-                              at most 3,670,016 triangles take tiles of
-                              their own
-                              (256 leaves, no climb) */
+                              256|512|1024.  Not fixed and with no HBM budget,
+                              builds and refits of at most 3,670,016 triangles
+                              (batches of as many in all) do not use it: they
+                              take tiles of their own (256 leaves, no climb) */
   LBVH_TUNE_SORT_BITS = 1  /* digit width of the builds' radix sort: 8 (4
                               passes over the 30-bit Morton keys) or 10 (3
                               passes); the reference uses 2-bit digits,
-                              radix-sort.js:486.  Not fixed, builds and
-                              sorts of at most 2^18 merge sorted tiles
-                              instead of radix passes */
+                              radix-sort.js:486.  Not fixed, single builds of at
+                              most 393,216 triangles and lbvh_sort of at most
+                              2^18 keys do not use it: they merge sorted
+                              tiles instead of radix passes */
 } lbvh_tunable;
 /* set_tuning fixes a value for every size (value 0: no fixed value, builds
  * use the autotuned table, else the size-based default: tree tile 1024, and
  * 10-bit digits up to 2^17 triangles and from 2^20 + 1 to 2^21, 8-bit
- * elsewhere); get_tuning_for returns
- * the value a build of n triangles would use (n = 0: the fixed/default
- * value). */
+ * elsewhere); get_tuning_for returns the value in force for n triangles
+ * (n = 0: the fixed/default value): what the builds of that size take that use
+ * the tunable (lbvh_tunable names those that do not). */
 int lbvh_set_tuning(lbvh_ctx *ctx, int param, int value);
 int lbvh_get_tuning(const lbvh_ctx *ctx, int param);
 int lbvh_get_tuning_for(const lbvh_ctx *ctx, int param, uint32_t n);
 /* Autotuner: for every power-of-two size bucket 2^k in [n_min, n_max] it
  * builds a device-synthesised uniform mesh of 2^k triangles with each
- * variant of every tunable, times them with HIP events (median of `reps`
- * after a warm-up) and keeps the fastest per bucket if it beats the
+ * variant of every tunable fixed (so with radix passes and the fused up pass
+ * also where unfixed builds take neither), times them with HIP events (median
+ * of `reps` after a warm-up) and keeps the fastest per bucket if it beats the
  * size-based default by more than 2 %, else the default; later builds pick the
  * entry of their size's bucket (or the nearest tuned one).  A fixed value
  * from lbvh_set_tuning is cleared.  ms_out (optional) receives, per bucket

@@ -47,7 +47,6 @@ struct lbvh_ctx {
   int tune_tile[33] = {0};       // autotuned tree tile per log2 size bucket
   int sort_bits = kRadixBits;    // sort digit width (8 or 10)
   bool sort_bits_fixed = false;
-  bool tuning = false;           // lbvh_autotune is timing its variants
   int tune_bits[33] = {0};       // autotuned digit width per size bucket
   std::string last_error;
   AllocTable user_allocs;  // buffers handed out by lbvh_alloc
@@ -505,7 +504,7 @@ int bits_for(const lbvh_ctx *ctx, uint32_t n) {
 // Whether a single-mesh sort of n keys (at most `most`) merges sorted tiles; a
 // fixed digit width asks for the radix passes.
 bool merge_sorted(const lbvh_ctx *ctx, uint32_t n, uint32_t most) {
-  return n <= most && !(ctx->sort_bits_fixed && !ctx->tuning);
+  return n <= most && !ctx->sort_bits_fixed;
 }
 
 // The key buffers of each pass of a sort from `in` to `out`: each pass reads
@@ -1089,9 +1088,11 @@ int lbvh_autotune(lbvh_ctx *ctx, uint32_t n_min, uint32_t n_max, int reps,
   (void)hipEventCreate(&b);
   const bool tile_was_fixed = ctx->tree_tile_fixed;
   const bool bits_were_fixed = ctx->sort_bits_fixed;
-  ctx->tree_tile_fixed = true;  // force each variant while timing
+  // Each variant is forced while it is timed, also at sizes whose builds merge or
+  // take k_forest.hip's leaf tiles: batches read the entries there, and larger
+  // sizes the nearest ones.
+  ctx->tree_tile_fixed = true;
   ctx->sort_bits_fixed = true;
-  ctx->tuning = true;
   const int saved_tile = ctx->tree_tile, saved_bits = ctx->sort_bits;
   int out_i = 0;
   st = LBVH_OK;
@@ -1139,7 +1140,6 @@ int lbvh_autotune(lbvh_ctx *ctx, uint32_t n_min, uint32_t n_max, int reps,
       ctx->tune_bits[k] = widths[pick % 2];
     }
   }
-  ctx->tuning = false;
   ctx->tree_tile = saved_tile;
   ctx->sort_bits = saved_bits;
   ctx->tree_tile_fixed = (st == LBVH_OK) ? false : tile_was_fixed;
