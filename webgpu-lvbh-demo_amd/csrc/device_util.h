@@ -93,15 +93,6 @@ __device__ __forceinline__ void store_nt(int4 *p, int4 v) {
   __builtin_nontemporal_store(nt_i4{v.x, v.y, v.z, v.w},
                               reinterpret_cast<nt_i4 *>(p));
 }
-typedef unsigned int nt_u4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ uint4 load_nt(const uint4 *p) {
-  const nt_u4 v = __builtin_nontemporal_load(reinterpret_cast<const nt_u4 *>(p));
-  return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ int4 load_nt(const int4 *p) {
-  const nt_i4 v = __builtin_nontemporal_load(reinterpret_cast<const nt_i4 *>(p));
-  return make_int4(v.x, v.y, v.z, v.w);
-}
 
 // Triangles in chunks of kMapThreads: a chunk's 3 * kMapThreads float4 are
 // loaded contiguously (each load instruction covers 4 KB, where a triangle

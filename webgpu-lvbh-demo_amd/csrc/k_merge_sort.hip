@@ -475,7 +475,7 @@ static int merge_plan(const MergeKeys &src, uint32_t n, MergeRound *r) {
   return rounds;
 }
 
-// Sample words of one buffer (merge_scratch_words holds two).
+// Sample words of one buffer; a sort's samples are two.
 static uint32_t merge_samples(uint32_t n) { return (n >> kSampleLog) + 1; }
 static_assert(kMergeBuildMax <= 16u << kMaxRunLog, "the last round's runs");
 static_assert(2 * ((kSmallSortTile >> kSampleLog) + 1) <= 2 * kRadix,

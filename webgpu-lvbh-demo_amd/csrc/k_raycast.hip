@@ -95,16 +95,17 @@ constexpr uint32_t kRayChunk = 64;  // consecutive blocks on one XCD
 //     mask, so addresses are selected, the far child is stored above the top
 //     whether it is pushed or not, the triangle test has no early ends, and
 //     one branch holds all of the stack past LDS.
-// Together 245 -> 172 us for a 512 x 512 frame over 100,000 clustered
-// triangles (186 before the last but one), 1,000 -> 740 us for 1M scattered rays over 1M;
-// the last by wall clock: that frame 222 -> 197, a 1,024 x 1,024 frame over a
-// heightfield of 500,000 250 -> 221, 2^14 scattered rays over 4,097 triangles 65
-// -> 54, 1M over 1M uniform 1,150 -> 1,131, 1M over a surface of 300,000 540 ->
-// 547.  Dropping popped nodes beyond the closest hit lost (the stack entries
+// Calls back to back in us, with a fetch per kind, blocks of 256 and the stack in
+// scratch memory / now: a 512 x 512 frame over 100,000 clustered triangles 286 /
+// 204, 1,024 x 1,024 over a heightfield of 300,000 261 / 152, 2^14 scattered rays over
+// 4,097 uniform triangles 81 / 50, 1M over 1M uniform 1,615 / 1,110, over a surface of
+// 300,000 647 / 550 (540 before the straight-line steps); 1M over 100 triangles lose,
+// 75.4 / 77.4, as there are more blocks.
+// Dropping popped nodes beyond the closest hit lost (the stack entries
 // double), and so did descending to a leaf per lane before any test, touching
 // both children ahead, a step that takes a leaf together with the node that
-// comes off the stack after it (the frame 244), and a higher priority for waves
-// with many steps (235).
+// comes off the stack after it (the first frame 222 -> 244), and a higher
+// priority for waves with many steps (235).
 __global__ __launch_bounds__(kRayThreads) void k_raycast(
     const int4 *__restrict__ nodes, const int4 *__restrict__ tri, uint32_t n,
     const float4 *__restrict__ rays, uint32_t count, float4 *__restrict__ hits,

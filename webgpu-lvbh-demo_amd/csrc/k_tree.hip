@@ -136,7 +136,7 @@ __global__ __launch_bounds__(kRtThreads) void k_rt_tiles(
   }
   if (tid == 0) s_nrec = 0;
   __syncthreads();
-  // Deltas, and per segment (wave w owns segments 16w .. 16w + 15, lane l
+  // Deltas, and per segment (wave w owns segments 4w .. 4w + 3, lane l
   // gap l of each) its bit planes and its minimum.  With lane u standing for
   // the value u, the planes give the mask of the segment's gaps below u:
   // the tables of its last and first such gap come from it, and it stays in

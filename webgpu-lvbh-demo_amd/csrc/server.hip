@@ -135,7 +135,7 @@ constexpr uint64_t kMeshBytesPerTri = 168;
 constexpr uint64_t kBuildScratchPerTri = 80;
 constexpr uint64_t kRefitScratchPerTri = 36;
 // plus what does not scale with n: the context's control block, the bounds
-// partials (80 KB with headroom), and tile tables rounded up to whole tiles
+// partials (20 KB with headroom), and tile tables rounded up to whole tiles
 constexpr uint64_t kSlotScratchFixed = 1ull << 20;
 
 struct Mesh {
