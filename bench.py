@@ -371,6 +371,8 @@ def main():
     ap.add_argument("--tree-tile", type=int, default=0,
                     help="leaves per block of the fused up pass (256/512/1024); "
                          "with --sort-bits, replaces the autotuner")
+    ap.add_argument("--no-autotune", action="store_true",
+                    help="build untuned (for profiles)")
     ap.add_argument("--sort-bits", type=int, default=0,
                     help="radix-sort digit width (8 or 10)")
     ap.add_argument("--no-batched", action="store_true")
@@ -413,7 +415,7 @@ def main():
             ctx.set_tuning(lb.TUNE_TREE_TILE, args.tree_tile)
         if args.sort_bits:
             ctx.set_tuning(lb.TUNE_SORT_BITS, args.sort_bits)
-    else:
+    elif not args.no_autotune:
         log("autotune")
         tuning = ctx.autotune(1 << 16, n, reps=3)
     d_tri = ctx.to_device(tri)
