@@ -25,7 +25,13 @@ __device__ __forceinline__ TileRange sort_tile_range(
     uint32_t tile_keys) {
   if (!segs.tile_seg) {
     const uint32_t b = tile * tile_keys;
-    return {b, min(b + tile_keys, n), 0u, n};
+    uint32_t end = min(b + tile_keys, n);
+    // A small tile's end stays scalar, and apart from a segment's.  Joined with
+    // that at one vector minimum, a tile waited there for its offsets, too, before
+    // it loaded its keys (sorts of 2^20 keys 76.4 us, 75.1 apart).  The large tile's
+    // kernels gain nothing and lose in batches (80M keys 5,477 -> 5,512).
+    if (tile_keys == (uint32_t)kSmallSortTile) asm("" : "+s"(end));
+    return {b, end, 0u, n};
   }
   const uint32_t sg = segs.tile_seg[tile];
   const uint32_t sb = segs.seg_off[sg], se = segs.seg_off[sg + 1];
