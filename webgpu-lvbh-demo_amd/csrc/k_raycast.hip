@@ -100,7 +100,8 @@ constexpr uint32_t kRayChunk = 64;  // consecutive blocks on one XCD
 // 204, 1,024 x 1,024 over a heightfield of 300,000 261 / 152, 2^14 scattered rays over
 // 4,097 uniform triangles 81 / 50, 1M over 1M uniform 1,615 / 1,110, over a surface of
 // 300,000 647 / 550 (540 before the straight-line steps); 1M over 100 triangles lose,
-// 75.4 / 77.4, as there are more blocks.
+// 75.4 / 77.4 (80 in blocks of 256): with the tree in L1 a step's instructions count,
+// and a straight-line step has more.
 // Dropping popped nodes beyond the closest hit lost (the stack entries
 // double), and so did descending to a leaf per lane before any test, touching
 // both children ahead, a step that takes a leaf together with the node that
